@@ -1,0 +1,35 @@
+// Host entry of the prompt-sized append (append_bulk.hip).
+#pragma once
+#include "append_row.h"
+
+namespace kvq {
+
+constexpr int kBulkMaxWaves = 8;      // waves per work-group at most
+constexpr int kBulkWaveSlots = 8192;  // most waves per side: 8 a SIMD on 256 CUs
+// Fewest new tokens per (b, head).  A wave takes 8 tokens at least, so below that lanes idle and
+// one row a wave is as good.
+constexpr int kBulkMinTokens = 8;
+// 32-token tiles per side from which a wave takes 32 (16) tokens, else 8: a longer tile has more
+// loads in flight, a shorter one gives more waves.  Measured in us for 8 / 16 / 32 tokens a wave:
+// 256 tiles (INT8, 2 x 4096 tokens) 5.4 / 5.8 / 7.9, 1024 (KIVI INT4, 4 x 8191) 21.2 / 12.5 / 12.5,
+// 1504 (INT4, 8 x 6001) 14.6 / 13.2 / 14.3.
+constexpr int kBulkTiles32 = 2048, kBulkTiles16 = 512;
+// tiles for which a work-group has 8 waves instead of 4 (INT4 with rescued groups, whose largest
+// value often counts as clipped, at 8 x 4096 tokens: 15.5 -> 13.0 us; 700 tiles of the mixed cache
+// 6.5 against 7.3 us, 32768 tiles of the asymmetric format 131 against 135 us)
+constexpr int kBulkWideFrom = 2048, kBulkWideTo = 8192;
+
+// Order statistics of a percentile (ranks and weight, as torch.quantile computes them) and
+// whether a static table has a per-token policy.
+struct BulkSide {
+  int top2, policy;
+  int lo, hi, blo, bhi;  // ranks near the top; KIVI V: near the bottom
+  float w, bw;
+};
+
+// Launches the tile kernel for the append of k and v if it takes both (else false, nothing
+// enqueued).  The caller has validated both sides (fill_dev) and filled thr_ptr where the group
+// rescue needs a threshold.
+bool append_bulk(const AppendDev& k, const AppendDev& v, hipStream_t st);
+
+}  // namespace kvq

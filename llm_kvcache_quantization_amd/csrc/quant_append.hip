@@ -13,6 +13,7 @@
 // Packing: byte = ((q[2i] + 8) << 4) | (q[2i+1] + 8)   src/quant/int4_basic.py:263-270
 // Divisions are IEEE fp32 (__fdiv_rn) and rounding is ties-to-even (rintf), which is
 // what torch does for tensor/tensor ops on both CPU and GPU.
+#include "append_bulk.h"
 #include "append_row.h"
 #include "kvq_common.h"
 #include "kvq.h"
@@ -437,6 +438,11 @@ extern "C" int kvq_quant_append(const kvq_append_params* k, const kvq_append_par
   if (!large && (needs_rescue(k) || needs_rescue(v))) {
     const int64_t nk = needs_rescue(k) ? rescue_n(k) : 0, nv = needs_rescue(v) ? rescue_n(v) : 0;
     rescue = (nk > nv ? nk : nv) <= kRescueRank ? 2 : 1;
+  }
+  if (rescue == 0 && append_bulk(dk, dv, s)) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(KVQ_ERR_LAUNCH, std::string("launch: ") + hipGetErrorString(e));
+    return KVQ_OK;
   }
   int64_t rows = 0;
   if (dk.valid) rows = (int64_t)dk.B * dk.H * dk.S;
