@@ -23,13 +23,15 @@ constexpr int kBulkWideFrom = 2048, kBulkWideTo = 8192;
 // whether a static table has a per-token policy.
 struct BulkSide {
   int top2, policy;
+  int local;             // the rescue threshold is found by the append's work-groups
   int lo, hi, blo, bhi;  // ranks near the top; KIVI V: near the bottom
   float w, bw;
 };
 
 // Launches the tile kernel for the append of k and v if it takes both (else false, nothing
-// enqueued).  The caller has validated both sides (fill_dev) and filled thr_ptr where the group
-// rescue needs a threshold.
-bool append_bulk(const AppendDev& k, const AppendDev& v, hipStream_t st);
+// enqueued).  The caller has validated both sides (fill_dev); a side's group rescue has its
+// threshold selected in its scratch, or with `local` (at most kRescueMax scales) every work-group
+// finds it.
+bool append_bulk(const AppendDev& k, const AppendDev& v, hipStream_t st, bool local);
 
 }  // namespace kvq

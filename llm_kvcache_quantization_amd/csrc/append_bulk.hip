@@ -18,8 +18,8 @@
 // RISC System/6000", 1990: a faithful q corrected with a correctly rounded r is RN(x / s)).  It
 // holds where nothing under- or overflows: tiles with a NaN or Inf, or a scale outside
 // [2^-30, 2^30], are left to the row quantizer after the wave's other tiles.
-#include "append_row.h"
 #include "append_bulk.h"
+#include "append_tile.h"
 
 #pragma clang fp contract(off)
 
@@ -27,21 +27,6 @@ namespace kvq {
 
 namespace {
 
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t pk_max_u(uint32_t a, uint32_t b) {
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a),
-                                                                __builtin_bit_cast(u16x2, b)));
-}
-__device__ __forceinline__ uint32_t pk_max_i(uint32_t a, uint32_t b) {
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(i16x2, a),
-                                                                __builtin_bit_cast(i16x2, b)));
-}
-__device__ __forceinline__ uint32_t pk_min_i(uint32_t a, uint32_t b) {
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(i16x2, a),
-                                                                __builtin_bit_cast(i16x2, b)));
-}
 // both halves shifted left by one (an fp16 value without its sign bit)
 __device__ __forceinline__ uint32_t pk_double(uint32_t a) {
   const u16x2 v = __builtin_bit_cast(u16x2, a);
@@ -53,12 +38,6 @@ __device__ __forceinline__ uint32_t sort_key2(uint32_t w) {
   const uint32_t s = __builtin_bit_cast(uint32_t, v >> 15);
   return w ^ (s & 0x7FFF7FFFu);
 }
-template <int CTRL>
-__device__ __forceinline__ uint32_t dppu(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
-}
-__device__ __forceinline__ uint32_t swap16(uint32_t x) { return (x >> 16) | (x << 16); }
-
 // The two largest 16-bit integers (with multiplicity) of a set, kept in both halves of m1 / m2.
 struct Top2 {
   uint32_t m1, m2;
@@ -79,17 +58,6 @@ __device__ __forceinline__ void top2_group(Top2& t, int gs) {
   if (gs >= 32) t.merge(dppu<0x4E>(t.m1), dppu<0x4E>(t.m2));     // quad_perm [2, 3, 0, 1]
   if (gs >= 64) t.merge(dppu<0x141>(t.m1), dppu<0x141>(t.m2));   // row_half_mirror
   if (gs >= 128) t.merge(dppu<0x140>(t.m1), dppu<0x140>(t.m2));  // row_mirror
-}
-__device__ __forceinline__ uint32_t max_group(uint32_t m, int gs) {
-  if (gs >= 16) m = pk_max_i(m, dppu<0xB1>(m));
-  if (gs >= 32) m = pk_max_i(m, dppu<0x4E>(m));
-  if (gs >= 64) m = pk_max_i(m, dppu<0x141>(m));
-  if (gs >= 128) m = pk_max_i(m, dppu<0x140>(m));
-  return m;
-}
-
-__device__ __forceinline__ float half_bits(uint32_t b) {
-  return (float)__builtin_bit_cast(half_t, (uint16_t)b);
 }
 // the value of a sort key (low half)
 __device__ __forceinline__ float key_value(uint32_t k) {
@@ -182,41 +150,51 @@ __device__ __forceinline__ int at_limit(u32x2 w) {
   return n;
 }
 
-// token of a tile that lane group g loads as its i-th: four whole rows an instruction; in the
-// TILE32 order the 8 tokens of a lane are those of its 32 bytes (tile32_offset)
-template <bool TILE>
-__device__ __forceinline__ constexpr int tok_of_i(int i) {
-  return TILE ? 16 * (i >> 2) + (i & 3) : 4 * i;
-}
-// a lane's 8 channels of a row; a side with outlier channels reads single values of the row
-// again, so its rows stay in the caches (streamed, they were fetched twice: 171 -> 131 us at
-// 8 x 4 heads x 32768 tokens)
-template <bool STREAM>
-__device__ __forceinline__ u32x4 ld_row(const half_t* p) {
-  const u32x4* q = reinterpret_cast<const u32x4*>(p);
-  if constexpr (STREAM) return __builtin_nontemporal_load(q);
-  return *q;
-}
-template <bool TILE>
-__device__ __forceinline__ int tok_of_g(int g) {
-  return TILE ? 4 * g : g;
-}
-
-// a lane's rows of the tile at prompt token s0; rows outside the prompt read its first / last row
-template <int NT, bool TILE, bool STREAM>
-__device__ __forceinline__ void load_tile(const AppendDev& a, const half_t* xr, int s0, int g, int d0,
-                                          bool full, u32x4 w[NT]) {
-  if (full) {  // lane base + uniform offsets
-    const half_t* xl = xr + (int64_t)(s0 + tok_of_g<TILE>(g)) * a.xss + d0;
-#pragma unroll
-    for (int i = 0; i < NT; ++i) w[i] = ld_row<STREAM>(xl + tok_of_i<TILE>(i) * a.xss);
-  } else {
-#pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      const int s = min(max(s0 + tok_of_g<TILE>(g) + tok_of_i<TILE>(i), 0), a.S - 1);
-      w[i] = ld_row<STREAM>(xr + (int64_t)s * a.xss + d0);
-    }
+// The threshold of a side of at most kRescueMax (row, group) scales, found by one work-group over
+// all rows (each work-group of the append finds it itself).
+struct LocalRescue {
+  uint32_t hist[256], bucket[2], rank[2];
+  uint16_t key[kRescueMax];
+};
+__device__ __forceinline__ float local_threshold(const AppendDev& a, LocalRescue& l) {
+  constexpr int NT = 4, kTok = 4 * NT;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, c = lane & 15, waves = blockDim.x >> 6, G = 128 / a.gs;
+  const int rows = a.B * a.H * a.S, n = rows * G;
+  for (int i = threadIdx.x; i < 256; i += blockDim.x) l.hist[i] = 0;
+  __syncthreads();
+  const int ntile = (a.S + kTok - 1) / kTok, items = a.B * a.H * ntile;
+  for (int item = wave; item < items; item += waves) {
+    const int bh = item / ntile, s0 = (item - bh * ntile) * kTok;
+    const half_t* xr = a.x + (int64_t)(bh / a.H) * a.xsb + (int64_t)(bh % a.H) * a.xsh;
+    u32x4 w[NT];
+    load_tile<NT, false, kCached>(a, xr, s0, g, 8 * c, s0 + kTok <= a.S, w);
+    tile_keys<NT>(a, w, s0, g, c, [&](int i, uint32_t key) {
+      l.key[(bh * a.S + s0 + 4 * i + g) * G + 8 * c / a.gs] = (uint16_t)key;
+      atomicAdd(&l.hist[key >> 7], 1u);
+    });
   }
+  __syncthreads();
+  if (wave == 0) {
+    uint32_t lo, hi, b, at;
+    float w;
+    quantile_ranks(a.rq, n, lo, hi, w);
+    bin_of_rank<4>(l.hist, lo, lane, b, at);
+    if (lane == 0) l.bucket[0] = b, l.rank[0] = at;
+    bin_of_rank<4>(l.hist, hi, lane, b, at);
+    if (lane == 0) l.bucket[1] = b, l.rank[1] = at;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 256; i += blockDim.x) l.hist[i] = 0;
+  const uint32_t b0 = l.bucket[0], b1 = l.bucket[1];
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    const uint32_t key = l.key[i];
+    if (key >> 7 == b0) atomicAdd(&l.hist[key & 127], 1u);
+    if (key >> 7 == b1) atomicAdd(&l.hist[128 + (key & 127)], 1u);
+  }
+  __syncthreads();
+  return rescue_threshold(a, l.hist, l.bucket, l.rank, lane);
 }
 
 // One side of the append: FMT its format, NT tokens per lane (4 NT per tile), TILE the TILE32
@@ -237,7 +215,15 @@ __device__ __forceinline__ void bulk_side(const AppendDev& a, const BulkSide& bs
   const int ntile = (lead + a.S + kTok - 1) / kTok;
   const int waves = blockDim.x >> 6;
   const int items = a.B * a.H * ntile, step = gridDim.x * waves;
-  const float thr = (FMT == KVQ_FMT_INT4_SYM && a.thr_ptr) ? *a.thr_ptr : 0.f;
+  float thr = 0.f;
+  if constexpr (FMT == KVQ_FMT_INT4_SYM) {
+    if (bs.local) {
+      __shared__ LocalRescue local;
+      thr = local_threshold(a, local);
+    } else if (const RescueScratch* sc = scratch_of(a)) {
+      thr = rescue_threshold(a, sc->hist, sc->bucket, sc->rank, lane);
+    }
+  }
   const bool table = a.st != nullptr;
   const bool outl = FMT == KVQ_FMT_INT4_ASYM && NT == 8 && a.n_out > 0;
   int clipped = 0;
@@ -249,8 +235,8 @@ __device__ __forceinline__ void bulk_side(const AppendDev& a, const BulkSide& bs
     const half_t* xr = a.x + (int64_t)b * a.xsb + (int64_t)h * a.xsh;
     const bool full = s0 >= 0 && s0 + kTok <= a.S;
     u32x4 w[NT];
-    if (outl) load_tile<NT, TILE, false>(a, xr, s0, g, d0, full, w);
-    else load_tile<NT, TILE, true>(a, xr, s0, g, d0, full, w);
+    if (outl) load_tile<NT, TILE, kCached>(a, xr, s0, g, d0, full, w);
+    else load_tile<NT, TILE, kStream>(a, xr, s0, g, d0, full, w);
     // outlier channels (INT4_ASYM K): lane l copies channels 2 (l % 2), + 1 of token l / 2
     uint32_t ov = 0;
     const int so = s0 + (lane >> 1);
@@ -592,11 +578,13 @@ int64_t tiles_of(const AppendDev& d, int tok) {
 
 }  // namespace
 
-bool append_bulk(const AppendDev& k, const AppendDev& v, hipStream_t st) {
+bool append_bulk(const AppendDev& k, const AppendDev& v, hipStream_t st, bool local) {
   BulkSide ks, vs;
   if (!side_ok(k, ks) || !side_ok(v, vs)) return false;
   const int s_new = k.valid ? k.S : v.S;
   if (s_new < kBulkMinTokens) return false;
+  ks.local = local && needs_threshold(k);
+  vs.local = local && needs_threshold(v);
   // a missing side runs as the other one's format (its work-groups exit at once)
   const int ck = k.valid ? side_code(k) : side_code(v), cv = v.valid ? side_code(v) : side_code(k);
   // 32 tokens a wave where that gives every SIMD a few waves, fewer in shorter prompts
@@ -607,7 +595,7 @@ bool append_bulk(const AppendDev& k, const AppendDev& v, hipStream_t st) {
   if (tiles > ((int64_t)1 << 30)) return false;
   // every work-group that clipped adds to one status word, and such atomics queue (about 10 ns
   // each): 8 waves a work-group where that counts and the tiles fill the SIMDs, else 4
-  const int waves = tiles >= kBulkWideFrom && tiles < kBulkWideTo ? 8 : 4;
+  const int waves = local || (tiles >= kBulkWideFrom && tiles < kBulkWideTo) ? 8 : 4;
   int64_t gx = (tiles + waves - 1) / waves;
   // at most 64 tiles a wave (its redo mask)
   const int64_t least = (tiles + 64 * waves - 1) / (64 * waves), most = kBulkWaveSlots / waves;

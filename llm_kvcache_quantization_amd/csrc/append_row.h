@@ -21,6 +21,7 @@ int fail(int code, const std::string& msg);
 // append kernel's work-groups, or the fused decode step's writer wave), walking down from the
 // maximum when its ranks lie within kTopWalk of the top; rows are loaded kRowBatch at a time.
 constexpr int kRescueRank = 1024;
+constexpr int kRescueMax = 4096;  // most (row, group) scales whose threshold needs no scratch
 constexpr int kRowBatch = 8;
 constexpr int kTopWalk = 32;
 
@@ -53,16 +54,10 @@ struct AppendDev {
   int tile32;  // codes in KVQ_LAYOUT_TILE32 (INT4_ASYM)
   float dq;              // dynamic scales: fp32(percentile / 100), or 0 for the absmax
   float dq_lo;           // KIVI V: fp32((100 - percentile) / 100), the low quantile
-  const float* thr_ptr;  // group-rescue threshold computed by the large-n select, or NULL
+  void* rescue;          // the group rescue's select over many scales (RescueScratch), or NULL
   int64_t st_sb;         // INT4_KIVI K: batch stride of the per-channel parameters
   float* zo;             // INT4_KIVI V: per-token zero-point out (scale_out's strides)
 };
-
-// Scratch of the group rescue over more than kRescueMax (row, group) scales: an exact radix
-// select, over the fp32 bit patterns of the append's dynamic group scales (all positive,
-// so their bit patterns sort as their values; a NaN sorts last as in torch.sort), of
-// sorted[lo] (4 histogram passes of 8 bits), then sorted[hi] (lo + 1) from the count of
-// values <= sorted[lo] and the least value above it, then torch.quantile's interpolation.
 
 __device__ __forceinline__ float ld_static(const AppendDev& a, int h, int g) {
 #pragma clang fp contract(off)
@@ -171,6 +166,11 @@ __device__ __forceinline__ float group_absmax(float v, int gs) {
   if (gs >= 64) v = fmaxf(v, __shfl_xor(v, 16, 64));
   if (gs >= 128) v = fmaxf(v, __shfl_xor(v, 32, 64));
   return v;
+}
+
+// whether a side's scales depend on the group rescue's threshold
+__host__ __device__ __forceinline__ bool needs_threshold(const AppendDev& a) {
+  return a.valid && a.fmt == KVQ_FMT_INT4_SYM && a.st != nullptr && a.rq > 0.f && !a.rescue_all;
 }
 
 // Scale of group g for a row, before the per-format final clamp.

@@ -15,6 +15,7 @@
 // what torch does for tensor/tensor ops on both CPU and GPU.
 #include "append_bulk.h"
 #include "append_row.h"
+#include "append_tile.h"
 #include "kvq_common.h"
 #include "kvq.h"
 
@@ -33,123 +34,68 @@ extern thread_local std::string g_last_error;
 int fail(int code, const std::string& msg);
 
 constexpr int kAppendWaves = 4;
-constexpr int kRescueMax = 4096;  // (rows x groups) handled by the single-work-group rescue path
 
-struct RescueScratch {
-  uint32_t hist[256];
-  uint32_t prefix;  // bits of sorted[lo] fixed so far (all 32 after the last pass)
-  uint32_t rank;    // rank of sorted[lo] among the values that match prefix
-  uint32_t cnt_le;  // number of values <= sorted[lo]
-  uint32_t min_gt;  // least bit pattern above sorted[lo]
-  float thr;
-  uint32_t pad[3];
-};
+// ---------------------------------------------------------------- rescue over many scales
+//
+// Five short launches for both sides together, the append included: clear, upper-bit histogram,
+// buckets, lower-bit histogram, append (append_tile.h).
 
-// Calls f(bits) for the fp32 bit pattern of the dynamic scale fmax(absmax, 1e-5) / 7 of every
-// (row, group) of the append (int4_cache.py:344-358), one wave per row, grid-stride.
-template <class F>
-__device__ __forceinline__ void for_each_dyn(const AppendDev& a, F f) {
+__global__ void rescue_clear_kernel(RescueScratch* k, RescueScratch* v) {
+  RescueScratch* s = blockIdx.x ? v : k;
+  if (s) s->hist[threadIdx.x] = 0;
+}
+
+// PASS 0: the histogram of the upper 8 bits; 1: of the lower 7 bits within both buckets
+template <int PASS, RowLoad LD>
+__device__ __forceinline__ void rescue_hist_side(const AppendDev& a, uint32_t* h) {
+  RescueScratch* const sc = scratch_of(a);
+  if (!sc) return;
+  constexpr int NT = 4, kTok = 4 * NT;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int rows = a.B * a.H * a.S;
-  for (int row = blockIdx.x * kAppendWaves + wave; row < rows; row += gridDim.x * kAppendWaves) {
-    const int s_idx = row % a.S, bh = row / a.S, h = bh % a.H, b = bh / a.H;
-    const half_t* xr = a.x + (int64_t)b * a.xsb + (int64_t)h * a.xsh + (int64_t)s_idx * a.xss;
-    const half2v xv = *reinterpret_cast<const half2v*>(xr + 2 * lane);
-    const float am = group_max(fmaxf(fabsf((float)xv.x), fabsf((float)xv.y)), a.gs);
-    if ((2 * lane) % a.gs == 0) f(__float_as_uint(__fdiv_rn(fmaxf(am, 1e-5f), 7.0f)));
-  }
-}
-
-// rank of torch.quantile's lower order statistic: lo = floor(fp32(q) * (n - 1)); hi = ceil
-__device__ __forceinline__ void quantile_ranks(float q, int64_t n, int64_t& lo, int64_t& hi, float& w) {
-  const float rank = q * (float)(n - 1);
-  lo = (int64_t)floorf(rank);
-  hi = (int64_t)ceilf(rank);
-  w = rank - (float)lo;
-}
-
-__global__ void rescue_init_kernel(RescueScratch* s, float q, int64_t n) {
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) s->hist[i] = 0;
-  if (threadIdx.x == 0) {
-    int64_t lo, hi;
-    float w;
-    quantile_ranks(q, n, lo, hi, w);
-    s->prefix = 0;
-    s->rank = (uint32_t)lo;
-    s->cnt_le = 0;
-    s->min_gt = 0xFFFFFFFFu;
-  }
-}
-
-// histogram of digit `pass` (bits [24 - 8 pass, 32 - 8 pass)) over the values whose higher
-// digits equal the prefix found so far
-__global__ __launch_bounds__(kAppendWaves * 64) void rescue_hist_kernel(AppendDev a, RescueScratch* s,
-                                                                         int pass) {
-  __shared__ uint32_t h[256];
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) h[i] = 0;
+  const int g = lane >> 4, c = lane & 15, waves = blockDim.x >> 6;
+  h[threadIdx.x] = 0;  // 256 threads
   __syncthreads();
-  const uint32_t pre = s->prefix;
-  const int sh = 24 - 8 * pass;
-  for_each_dyn(a, [&](uint32_t bits) {
-    if (pass == 0 || (bits >> (sh + 8)) == (pre >> (sh + 8))) atomicAdd(&h[(bits >> sh) & 255u], 1u);
-  });
-  __syncthreads();
-  for (int i = threadIdx.x; i < 256; i += blockDim.x)
-    if (h[i]) atomicAdd(&s->hist[i], h[i]);
-}
-
-// picks the digit whose bucket holds the remaining rank, and clears the histogram
-__global__ void rescue_select_kernel(RescueScratch* s, int pass) {
-  __shared__ uint32_t digit, before;
-  if (threadIdx.x == 0) {
-    uint32_t cum = 0, d = 255, r = s->rank;
-    for (uint32_t i = 0; i < 256; ++i) {
-      const uint32_t c = s->hist[i];
-      if (r < cum + c) {
-        d = i;
-        break;
+  const uint32_t b0 = PASS ? sc->bucket[0] : 0, b1 = PASS ? sc->bucket[1] : 0;
+  const int ntile = (a.S + kTok - 1) / kTok, items = a.B * a.H * ntile;
+  for (int item = blockIdx.x * waves + wave; item < items; item += gridDim.x * waves) {
+    const int bh = item / ntile, s0 = (item - bh * ntile) * kTok;
+    const half_t* xr = a.x + (int64_t)(bh / a.H) * a.xsb + (int64_t)(bh % a.H) * a.xsh;
+    u32x4 w[NT];
+    load_tile<NT, false, LD>(a, xr, s0, g, 8 * c, s0 + kTok <= a.S, w);
+    tile_keys<NT>(a, w, s0, g, c, [&](int, uint32_t key) {
+      if (PASS == 0) {
+        atomicAdd(&h[key >> 7], 1u);
+      } else {
+        if (key >> 7 == b0) atomicAdd(&h[key & 127], 1u);
+        if (key >> 7 == b1) atomicAdd(&h[128 + (key & 127)], 1u);
       }
-      cum += c;
-    }
-    digit = d;
-    before = cum;
+    });
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) s->hist[i] = 0;
-  if (threadIdx.x == 0) {
-    s->prefix |= digit << (24 - 8 * pass);
-    s->rank -= before;
-  }
+  if (h[threadIdx.x]) atomicAdd(&sc->hist[threadIdx.x], h[threadIdx.x]);
+}
+template <int PASS, RowLoad LD>
+__global__ __launch_bounds__(256) void rescue_hist_kernel(AppendDev k, AppendDev v) {
+  __shared__ uint32_t h[256];
+  rescue_hist_side<PASS, LD>(blockIdx.y ? v : k, h);
 }
 
-// number of values <= sorted[lo] and the least value above it
-__global__ __launch_bounds__(kAppendWaves * 64) void rescue_count_kernel(AppendDev a, RescueScratch* s) {
-  __shared__ uint32_t cnt, mn;
-  if (threadIdx.x == 0) {
-    cnt = 0;
-    mn = 0xFFFFFFFFu;
+// the buckets of both ranks; clears the histogram.  One work-group of 256 threads a side.
+__global__ __launch_bounds__(256) void rescue_bucket_kernel(AppendDev k, AppendDev v) {
+  const AppendDev& a = blockIdx.x ? v : k;
+  RescueScratch* const sc = scratch_of(a);
+  if (!sc) return;
+  if (threadIdx.x < 64) {
+    uint32_t lo, hi, b, at;
+    float w;
+    quantile_ranks(a.rq, (int64_t)a.B * a.H * a.S * (128 / a.gs), lo, hi, w);
+    bin_of_rank<4>(sc->hist, lo, threadIdx.x, b, at);
+    if (threadIdx.x == 0) sc->bucket[0] = b, sc->rank[0] = at;
+    bin_of_rank<4>(sc->hist, hi, threadIdx.x, b, at);
+    if (threadIdx.x == 0) sc->bucket[1] = b, sc->rank[1] = at;
   }
   __syncthreads();
-  const uint32_t lo_bits = s->prefix;
-  for_each_dyn(a, [&](uint32_t bits) {
-    if (bits <= lo_bits) atomicAdd(&cnt, 1u);
-    else atomicMin(&mn, bits);
-  });
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    if (cnt) atomicAdd(&s->cnt_le, cnt);
-    if (mn != 0xFFFFFFFFu) atomicMin(&s->min_gt, mn);
-  }
-}
-
-// torch.quantile's interpolation of sorted[lo] and sorted[hi] (sorted_quantile's arithmetic)
-__global__ void rescue_thr_kernel(RescueScratch* s, float q, int64_t n) {
-  int64_t lo, hi;
-  float w;
-  quantile_ranks(q, n, lo, hi, w);
-  const float va = __uint_as_float(s->prefix);
-  const float vb = (hi < (int64_t)s->cnt_le) ? va : __uint_as_float(s->min_gt);
-  s->thr = quantile_lerp(va, vb, w);
+  sc->hist[threadIdx.x] = 0;
 }
 
 __device__ __forceinline__ void quant_row(const AppendDev& a, int row, int lane, float thr) {
@@ -229,9 +175,10 @@ __device__ __forceinline__ void append_side(const AppendDev& a, int rescue) {
   // scalar unit, not as vector integer division in every lane
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rows = a.B * a.H * a.S;
-  float thr = a.thr_ptr ? *a.thr_ptr : 0.f;
+  float thr = 0.f;
+  if (const RescueScratch* sc = scratch_of(a)) thr = rescue_threshold(a, sc->hist, sc->bucket, sc->rank, lane);
   __shared__ float dyn[kRescueMax];
-  const bool resc_side = a.fmt == KVQ_FMT_INT4_SYM && a.st != nullptr && a.rq > 0.f && !a.rescue_all;
+  const bool resc_side = needs_threshold(a);
   if (rescue == 2 && resc_side) {
     // Global threshold over every (row, group) dynamic scale of this append
     // (int4_cache.py:384-389), found by each work-group over all rows (n <= kRescueRank):
@@ -387,28 +334,41 @@ static int64_t rescue_n(const kvq_append_params* p) {
   return (int64_t)p->batch * p->heads * p->seq_new * (128 / p->group_size);
 }
 
-// the threshold of p's group rescue over more than kRescueMax scales, into its scratch
-static int rescue_large(const kvq_append_params* p, AppendDev& d, const char* name, hipStream_t st) {
+// checks p's scratch and gives it to d
+static int take_scratch(const kvq_append_params* p, AppendDev& d, const char* name) {
   const std::string n(name);
   if (!p->scratch || p->scratch_bytes < (int64_t)sizeof(RescueScratch) || ((uintptr_t)p->scratch % 16))
     return fail(KVQ_ERR_INVALID, n + ": outlier rescue over more than 4096 (row, group) scales needs "
                                      "a 16-byte aligned scratch of kvq_append_scratch_bytes() bytes");
-  RescueScratch* s = reinterpret_cast<RescueScratch*>(p->scratch);
-  const int64_t cnt = rescue_n(p);
-  if (cnt >= ((int64_t)1 << 31)) return fail(KVQ_ERR_UNSUPPORTED, n + ": too many (row, group) scales");
-  const int64_t rows = (int64_t)p->batch * p->heads * p->seq_new;
-  int64_t gx = (rows + kAppendWaves - 1) / kAppendWaves;
-  if (gx > 2048) gx = 2048;
-  const dim3 grid((unsigned)gx), block(kAppendWaves * 64);
-  hipLaunchKernelGGL(rescue_init_kernel, dim3(1), dim3(256), 0, st, s, p->rescue_quantile, cnt);
-  for (int pass = 0; pass < 4; ++pass) {
-    hipLaunchKernelGGL(rescue_hist_kernel, grid, block, 0, st, d, s, pass);
-    hipLaunchKernelGGL(rescue_select_kernel, dim3(1), dim3(256), 0, st, s, pass);
-  }
-  hipLaunchKernelGGL(rescue_count_kernel, grid, block, 0, st, d, s);
-  hipLaunchKernelGGL(rescue_thr_kernel, dim3(1), dim3(1), 0, st, s, p->rescue_quantile, cnt);
-  d.thr_ptr = &s->thr;
+  if (rescue_n(p) >= ((int64_t)1 << 31)) return fail(KVQ_ERR_UNSUPPORTED, n + ": too many (row, group) scales");
+  d.rescue = p->scratch;
   return KVQ_OK;
+}
+
+template <RowLoad LD>
+static void rescue_select(const AppendDev& k, const AppendDev& v, unsigned gx, hipStream_t st) {
+  hipLaunchKernelGGL((rescue_hist_kernel<0, LD>), dim3(gx, 2), dim3(256), 0, st, k, v);
+  hipLaunchKernelGGL(rescue_bucket_kernel, dim3(2), dim3(256), 0, st, k, v);
+  hipLaunchKernelGGL((rescue_hist_kernel<1, LD>), dim3(gx, 2), dim3(256), 0, st, k, v);
+}
+
+// the select of both sides' thresholds into their scratches
+static void rescue_large(const AppendDev& k, const AppendDev& v, hipStream_t st) {
+  int64_t tiles = 0;
+  bool al16 = true;
+  for (const AppendDev* d : {&k, &v}) {
+    if (!d->rescue) continue;
+    const int64_t t = (int64_t)d->B * d->H * ((d->S + 15) / 16);
+    tiles = tiles > t ? tiles : t;
+    al16 = al16 && (uintptr_t)d->x % 16 == 0 && d->xsb % 8 == 0 && d->xsh % 8 == 0 && d->xss % 8 == 0;
+  }
+  // a work-group's histogram costs up to 256 global atomics, so a few tiles a wave
+  int64_t gx = (tiles + 15) / 16;
+  gx = gx < 1 ? 1 : gx > 512 ? 512 : gx;
+  hipLaunchKernelGGL(rescue_clear_kernel, dim3(2), dim3(256), 0, st, reinterpret_cast<RescueScratch*>(k.rescue),
+                     reinterpret_cast<RescueScratch*>(v.rescue));
+  if (al16) rescue_select<kCached>(k, v, (unsigned)gx, st);
+  else rescue_select<kDwords>(k, v, (unsigned)gx, st);
 }
 
 }  // namespace kvq
@@ -429,17 +389,19 @@ extern "C" int kvq_quant_append(const kvq_append_params* k, const kvq_append_par
   const bool large = (needs_rescue(k) && rescue_n(k) > kRescueMax) ||
                      (needs_rescue(v) && rescue_n(v) > kRescueMax);
   if (large) {
-    if (needs_rescue(k) && (rc = rescue_large(k, dk, "k", s))) return rc;
-    if (needs_rescue(v) && (rc = rescue_large(v, dv, "v", s))) return rc;
+    if (needs_rescue(k) && (rc = take_scratch(k, dk, "k"))) return rc;
+    if (needs_rescue(v) && (rc = take_scratch(v, dv, "v"))) return rc;
+    rescue_large(dk, dv, s);
   }
-  // decode-sized rescues (at most kRescueRank scales per side): every work-group finds the
-  // threshold; else one work-group does
+  // rescues over at most kRescueMax scales: a prompt's tile kernel finds the threshold in every
+  // work-group (4 heads x 103 tokens in groups of 16: 267 -> 12 us, 2 x 60: 21.5 -> 8.8 us), the
+  // row kernel in every work-group up to kRescueRank scales (decode steps), else in one
   int rescue = 0;
   if (!large && (needs_rescue(k) || needs_rescue(v))) {
     const int64_t nk = needs_rescue(k) ? rescue_n(k) : 0, nv = needs_rescue(v) ? rescue_n(v) : 0;
     rescue = (nk > nv ? nk : nv) <= kRescueRank ? 2 : 1;
   }
-  if (rescue == 0 && append_bulk(dk, dv, s)) {
+  if (append_bulk(dk, dv, s, rescue != 0)) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(KVQ_ERR_LAUNCH, std::string("launch: ") + hipGetErrorString(e));
     return KVQ_OK;

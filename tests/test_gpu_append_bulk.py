@@ -71,17 +71,23 @@ def _side(C, fmt, gs, B, H, S, wpos, cap, x, policy, g, tile=False):
             p.static_zp = z.data_ptr()
             keep.append(z)
     p.adaptive, p.adaptive_margin = int("margin" in policy), policy.get("margin", 0.0)
+    p.rescue_quantile = policy.get("rq", 0.0)
     p.mixed_rescue, p.rescue_all = int(policy.get("mixed", 0)), int(policy.get("all", 0))
     if "pct" in policy:
         p.dyn_quantile = policy["pct"] / 100.0
     if fmt != C.KVQ_FMT_INT4_ASYM and (not policy.get("table") or "margin" in policy or policy.get("mixed")
-                                       or policy.get("all")):
+                                       or policy.get("all") or "rq" in policy):
         dt = torch.float16 if fmt == C.KVQ_FMT_INT8_SYM else torch.float32
         so = torch.full((B, H, cap, G), 7.0, dtype=dt, device="cuda")
         p.scale_out = so.data_ptr()
         p.scale_out_dtype = C.KVQ_DTYPE_F16 if dt == torch.float16 else C.KVQ_DTYPE_F32
         p.so_stride_b, p.so_stride_h, p.so_stride_t, p.so_stride_g = so.stride()
         out.append(so)
+    nbytes = C.lib().kvq_append_scratch_bytes(ctypes.byref(p))
+    if nbytes:
+        sc = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device="cuda")
+        p.scratch, p.scratch_bytes = sc.data_ptr(), nbytes
+        keep.append(sc)
     if policy.get("outliers"):
         oi = torch.stack([torch.randperm(D, generator=g, device="cuda")[:4] for _ in range(H)]).int()
         oo = torch.full((B, H, cap, 4), 7.0, dtype=torch.float16, device="cuda")
@@ -105,6 +111,9 @@ PAIRS = {
     "int4_max_g8": ((I4, 8, {}),) * 2,
     "int4_table_mixed": ((I4, 32, dict(table=1, mixed=1)), (I4, 32, dict(table=1))),
     "int4_table_all": ((I4, 64, dict(table=1, all=1)), (I4, 64, dict(table=1, margin=0.8))),
+    "int4_rescue_g16": ((I4, 16, dict(table=1, rq=0.99)), (I4, 16, dict(table=1, rq=0.4))),
+    "int4_rescue_g8": ((I4, 8, dict(table=1, rq=0.999, margin=0.7)), (I4, 8, dict(table=1))),
+    "int4_rescue_nan": ((I4, 32, dict(table=1, rq=0.5, odd=1)),) * 2,
     "asym_tile": ((A4, 32, dict(table=1, outliers=1)), (A4, 32, dict(table=1), True)),
     "asym_odd": ((A4, 32, dict(table=1, odd=1)), (A4, 32, dict(table=1, odd=1), True)),
     "k8_asym": ((I8, 32, dict(table=1)), (A4, 32, dict(table=1), True)),
@@ -118,8 +127,9 @@ PAIRS = {
     "mixed48": ((K4, 32, dict(pct=99.9)), (I8, 32, dict(pct=99.9))),
 }
 
-# (batch, heads, tokens, write position): fewest tokens, a tile's edges, starts inside a tile, and
-# enough tiles for 32 tokens a wave in every format
+# (batch, heads, tokens, write position): fewest tokens, a tile's edges, starts inside a tile, a
+# size whose rescue threshold every work-group finds (1025 to 4096 scales), and enough tiles for
+# 32 tokens a wave in every format
 SIZES = [(1, 2, 8, 0), (2, 3, 31, 5), (1, 1, 33, 31), (3, 2, 64, 32), (2, 8, 4099, 1)]
 
 
