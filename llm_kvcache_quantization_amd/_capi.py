@@ -182,6 +182,10 @@ def lib() -> ctypes.CDLL:
         L.kvq_last_error.restype = ctypes.c_char_p
         L.kvq_abi_version.argtypes = []
         L.kvq_abi_version.restype = c_i32
+        # the engines' own entry points (csrc/engine_ops.h), no part of the public ABI
+        L.kvq_kivi_channel_range.argtypes = [c_vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_i32, c_i32,
+                                             c_f32, c_f32, c_vp, c_vp, c_vp]
+        L.kvq_kivi_channel_range.restype = c_i32
         ver = L.kvq_abi_version()
         if ver != ABI_VERSION:
             raise ImportError(f"{LIB_PATH} has ABI {ver}, this package needs {ABI_VERSION}; rebuild it")

@@ -1209,9 +1209,19 @@ def kivi_channel_params(k: Tensor, bits: int, percentile: float) -> Tuple[Tensor
     """Per-channel K scale / zero-point over the tokens of a prefill k [B, H, S, D]
     (quantize_asymmetric_per_channel, src/quant/asymmetric_quant.py:24-141, 199-224): the
     range (min / max, or the two quantiles) in fp32, floored at max(1e-5, fp16 tiny x
-    (qmax - qmin)), divided by qmax - qmin; z = min - qmin s.  fp32 [B, H, D]."""
+    (qmax - qmin)), divided by qmax - qmin; z = min - qmin s.  fp32 [B, H, D].  One HIP launch
+    for fp16 rows on the GPU (kvq_kivi_channel_range)."""
     qmin, qmax = (-8, 7) if bits == 4 else (-128, 127)
     lo_q, hi_q = _kivi_levels(percentile)
+    if (k.is_cuda and k.dtype == torch.float16 and k.ndim == 4 and k.shape[-1] == 128 and k.shape[2] > 0
+            and k.stride(-1) == 1 and k.data_ptr() % 4 == 0 and not any(s % 2 for s in k.stride()[:3])):
+        B, H, S, D = k.shape
+        s = torch.empty(B, H, D, dtype=torch.float32, device=k.device)
+        z = torch.empty_like(s)
+        C.check(C.lib().kvq_kivi_channel_range(k.data_ptr(), *k.stride()[:3], B, H, S, bits, lo_q, hi_q,
+                                               s.data_ptr(), z.data_ptr(),
+                                               ctypes.c_void_p(C.stream_handle(k.device))))
+        return s, z
     kf = k.float()
     if hi_q > 0.0:
         srt = torch.sort(kf, dim=2).values
@@ -1235,8 +1245,7 @@ class _KiviFamily(_EngineBase):
     parameters); a 16-bit side keeps fp16 values.  Codes: 4 bits packed [B, H, T, 64] (byte =
     ((c[2i]+8) << 4) | (c[2i+1]+8)), 8 bits int8 [B, H, T, 128].  Every quantized token goes
     through kvq_quant_append (HIP; per-token percentile clipping in the kernel); the prefill's
-    per-channel K range is reduced with torch (aminmax, or a sort and torch.lerp for a
-    percentile, as torch.quantile does).  Decode attention reads the cache in place through the
+    per-channel K range is one HIP launch (:func:`kivi_channel_params`).  Decode attention reads the cache in place through the
     tiled kernel of the layer's pair (kvq_decode_attn), the fp16 residual window (residual_length
     > 0) with it, merged by the kernel's merging work-group.
     """
@@ -1364,8 +1373,8 @@ class _KiviFamily(_EngineBase):
                 self._oor_step_counter += 1
             oor_check = self._oor_step_counter % self._oor_check_interval == 0
         if prefill:
-            if self.check_numerics and not bool(torch.isfinite(k).all()):
-                raise ValueError("quantize_asymmetric: input contains NaN or Inf")
+            # a NaN / Inf is found by the append's status word below, which then undoes this
+            before = self._k_scale[layer_id], self._k_zp[layer_id]
             self._k_scale[layer_id], self._k_zp[layer_id] = kivi_channel_params(k, kb, self.k_percentile)
             self._k_scale_initialized[layer_id] = True
         if kb != 16:
@@ -1405,6 +1414,10 @@ class _KiviFamily(_EngineBase):
                                              ctypes.c_void_p(C.stream_handle(k.device))))
         if status is not None:
             st = self._read_status()
+            if prefill and st[0] & 1:
+                self._k_scale[layer_id], self._k_zp[layer_id] = before
+                self._k_scale_initialized[layer_id] = False
+                raise ValueError("quantize_asymmetric: input contains NaN or Inf")
             if st[0] & 1 or st[2] & 1:
                 raise ValueError(f"KIVI append: {'K' if st[0] & 1 else 'V'} input contains NaN or Inf "
                                  "— refusing to quantize corrupt data")

@@ -28,6 +28,11 @@ template <int CTRL>
 __device__ __forceinline__ uint32_t dppu(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
 }
+// the value of the lane CTRL - 0x110 below in its row of 16, 0 past the row's start
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_shr(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);
+}
 __device__ __forceinline__ uint32_t swap16(uint32_t x) { return (x >> 16) | (x << 16); }
 
 __device__ __forceinline__ uint32_t max_group(uint32_t m, int gs) {
@@ -125,11 +130,15 @@ __device__ __forceinline__ void bin_of_rank(const uint32_t* h, uint32_t r, int l
   uint32_t v[R], sum = 0;
 #pragma unroll
   for (int i = 0; i < R; ++i) sum += v[i] = h[R * lane + i];
+  // inclusive prefix sum over the wave: within rows of 16 by DPP, then the row totals
   uint32_t upto = sum;
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t u = __shfl_up(upto, o, 64);
-    if (lane >= o) upto += u;
-  }
+  upto += dpp_shr<0x111>(upto);  // row_shr:1
+  upto += dpp_shr<0x112>(upto);
+  upto += dpp_shr<0x114>(upto);
+  upto += dpp_shr<0x118>(upto);
+  const uint32_t r0 = __builtin_amdgcn_readlane(upto, 15), r1 = r0 + __builtin_amdgcn_readlane(upto, 31),
+                 r2 = r1 + __builtin_amdgcn_readlane(upto, 47);
+  upto += lane < 16 ? 0u : lane < 32 ? r0 : lane < 48 ? r1 : r2;
   const uint64_t past = __ballot(r < upto);  // lanes whose bins reach past r
   const int owner = past ? __builtin_ctzll(past) : 63;
   uint32_t cum = upto - sum, b = R * lane, at = 0;
@@ -143,8 +152,8 @@ __device__ __forceinline__ void bin_of_rank(const uint32_t* h, uint32_t r, int l
     }
     cum += v[i];
   }
-  bin = __shfl(b, owner, 64);
-  within = __shfl(at, owner, 64);
+  bin = __builtin_amdgcn_readlane(b, owner);
+  within = __builtin_amdgcn_readlane(at, owner);
 }
 
 // rank of torch.quantile's lower order statistic: lo = floor(fp32(q) * (n - 1)); hi = ceil

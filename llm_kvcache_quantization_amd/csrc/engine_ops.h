@@ -1,0 +1,24 @@
+// Entry points of libkvq.so for this package's cache engines (llm_kvcache_quantization_amd/cache.py).
+// They are no part of the public C ABI (include/kvq.h) and may change with the engines.  The same
+// rules hold: plain device pointers, nothing allocates or synchronises, work goes to `stream`,
+// KVQ_OK or a KVQ_ERR_* code with kvq_last_error().
+#pragma once
+#include "kvq.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+// Per-channel scale and zero-point of a prompt's K for the KIVI layout
+// (quantize_asymmetric_per_channel, src/quant/asymmetric_quant.py:24-141, 199-224): over the S
+// tokens of x fp16 [B, H, S, 128] (strides in elements, channels contiguous, 4-byte aligned
+// rows), the minimum and maximum (q_hi = 0) or torch.quantile at the levels q_lo, q_hi, then
+// s = max(range, max(1e-5, 2^-14 span)) / span with span = 15 (bits 4) or 255 (bits 8), and
+// z = min + (span + 1) / 2 s; fp32 [B, H, 128] dense.
+int kvq_kivi_channel_range(const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_s, int32_t batch,
+                           int32_t heads, int32_t tokens, int32_t bits, float q_lo, float q_hi, float* scale,
+                           float* zero_point, kvq_stream_t stream);
+
+#ifdef __cplusplus
+}
+#endif

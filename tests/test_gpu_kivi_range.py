@@ -1,0 +1,82 @@
+"""The HIP per-channel range of a KIVI prompt (csrc/kivi_range.hip): bit-exact against the oracle's
+quantize_asymmetric_per_channel (torch.quantile on the CPU), at the edges of the rows a thread holds
+(2048 for 4 waves, 8192 for 16), for few and many (b, head) units, transposed and odd strides, ties
+and subnormals; and the torch path's handling of NaN / Inf."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _k(B, H, S, seed):
+    g = torch.Generator().manual_seed(seed)
+    k = torch.randn(B, H, S, 128, generator=g).half()
+    k[..., 5] *= 100
+    k[..., 17] = torch.randint(-2, 3, k[..., 17].shape, generator=g).half()   # ties
+    k[..., 31] *= 2.0 ** -20                                                    # subnormals
+    k[..., 40] = 0.0
+    k[..., 41] = -0.0
+    k[..., 63] = -k[..., 63].abs()
+    return k
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("pct", [100.0, 99.9, 97.3, 51.0])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 2, 2), (2, 5, 37), (1, 2, 2048), (1, 1, 2049), (3, 3, 700),
+                                   (1, 1, 8192), (1, 1, 8193), (1, 1, 17001)], ids=str)
+def test_channel_range_bitexact(shape, pct, bits):
+    from llm_kvcache_quantization_amd.cache import kivi_channel_params
+    from oracle import quant as OQ
+
+    k = _k(*shape, seed=shape[2])
+    _, rs, rz = OQ.quantize_asymmetric_per_channel(k, bits, pct)
+    s, z = kivi_channel_params(k.cuda(), bits, pct)
+    assert torch.equal(s.cpu(), rs) and torch.equal(z.cpu(), rz)
+
+
+@pytest.mark.parametrize("pct", [100.0, 99.9])
+def test_channel_range_strides(pct):
+    from llm_kvcache_quantization_amd.cache import kivi_channel_params
+
+    k = _k(2, 3, 501, 1).cuda()
+    ref = kivi_channel_params(k, 4, pct)
+    t = k.transpose(1, 2).contiguous().transpose(1, 2)               # [B, S, H, D] storage
+    odd = torch.zeros(2, 3, 501, 130, dtype=torch.float16, device="cuda")[..., 2:]
+    odd.copy_(k)                                                     # rows aligned to 4 bytes only
+    odd1 = torch.zeros(2, 3, 501, 131, dtype=torch.float16, device="cuda")[..., 1:129]
+    odd1.copy_(k)                                                    # to 2 bytes: the torch path
+    for x in (t, odd, odd1):
+        for a, b in zip(kivi_channel_params(x, 4, pct), ref):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("pct", [100.0, 99.0])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_channel_range_not_finite(bad, pct):
+    """Without check_numerics: as torch's aminmax / sort and lerp, which keep a NaN range."""
+    from llm_kvcache_quantization_amd.cache import kivi_channel_params
+
+    k = _k(1, 2, 300, 2)
+    k[0, 1, 7, 3] = k[0, 0, 250:, 9] = bad
+    got = kivi_channel_params(k.cuda(), 8, pct)
+    want = kivi_channel_params(k, 8, pct)
+    for a, b in zip(got, want):
+        assert torch.equal(a.cpu().nan_to_num(7e30, 8e30, -8e30), b.nan_to_num(7e30, 8e30, -8e30))
+
+
+def test_prefill_rejects_nan_and_keeps_no_parameters():
+    from llm_kvcache_quantization_amd import KIVIStyleKVCache
+
+    cache = KIVIStyleKVCache(1, quant_bits=4)
+    k = _k(1, 2, 40, 3).cuda()
+    bad = k.clone()
+    bad[0, 1, 20, 100] = float("nan")
+    with pytest.raises(ValueError, match="quantize_asymmetric: input contains NaN or Inf"):
+        cache.append(0, bad, k)
+    assert cache.get_seq_len() == 0 and cache._k_scale[0] is None and not cache._k_scale_initialized[0]
+    with pytest.raises(ValueError, match="V input contains NaN or Inf"):
+        cache.append(0, k, bad)
+    assert cache.get_seq_len() == 0
+    cache.clear()
+    cache.append(0, k, k)
+    assert cache.get_seq_len() == 40
