@@ -1613,7 +1613,9 @@ class _KiviFamily(_EngineBase):
         self._discard_step_status()
         self._layer_seq_lens = [0] * self.num_layers
         self._seq_len = 0
+        # the next prompt has parameters of its own
         self._steps = [None] * self.num_layers
+        self._apps = [None] * self.num_layers
         self._k_scale_initialized = [False] * self.num_layers
         self._k_scale = [None] * self.num_layers
         self._k_zp = [None] * self.num_layers
