@@ -186,6 +186,9 @@ def lib() -> ctypes.CDLL:
         L.kvq_kivi_channel_range.argtypes = [c_vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_i32, c_i32,
                                              c_f32, c_f32, c_vp, c_vp, c_vp]
         L.kvq_kivi_channel_range.restype = c_i32
+        pv = ctypes.POINTER(KvView)
+        L.kvq_dequant.argtypes = [pv, c_i32, c_i32, c_vp, pv, c_i32, c_i32, c_vp, c_i32, c_i32, c_i32, c_vp]
+        L.kvq_dequant.restype = c_i32
         ver = L.kvq_abi_version()
         if ver != ABI_VERSION:
             raise ImportError(f"{LIB_PATH} has ABI {ver}, this package needs {ABI_VERSION}; rebuild it")

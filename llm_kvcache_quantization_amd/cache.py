@@ -616,6 +616,13 @@ class _SymCacheBase(_EngineBase):
         return kc, vc, sv(self._k_scale[layer_id], self._k_tok[layer_id]), \
             sv(self._v_scale[layer_id], self._v_tok[layer_id])
 
+    def _dequant_sym(self, kc, vc, ks, vs):
+        """fp16 K, V of the views ``_raw_views`` returns, in one HIP launch."""
+        from .kernels import kv_view_tok
+
+        gs = self.group_size
+        return _dequant((kv_view_tok(kc, ks), self._fmt, gs), (kv_view_tok(vc, vs), self._fmt, gs), kc)
+
     def clear(self) -> None:
         self._discard_step_status()
         self._layer_seq_lens = [0] * self.num_layers
@@ -716,6 +723,8 @@ class INT8KVCache(_SymCacheBase):
         kc, vc, ks, vs = self._raw_views(layer_id)
         if kc.shape[2] == 0:
             logger.warning("get_kv(layer_id=%d) returning zero-length tensors.", layer_id)
+        if self.dtype == torch.float16:
+            return self._dequant_sym(kc, vc, ks, vs)
         return _deq_sym(kc, ks).to(self.dtype), _deq_sym(vc, vs).to(self.dtype)
 
     @classmethod
@@ -849,6 +858,8 @@ class INT4KVCache(_SymCacheBase):
 
     def get_kv(self, layer_id: int) -> Tuple[Tensor, Tensor]:
         kc, vc, ks, vs = self._raw_views(layer_id)
+        if self.dtype == torch.float16:
+            return self._dequant_sym(kc, vc, ks, vs)
         return (_deq_sym(_unpack(kc), ks).to(self.dtype), _deq_sym(_unpack(vc), vs).to(self.dtype))
 
     @classmethod
@@ -875,6 +886,20 @@ def _deq_sym(q: Tensor, s: Tensor) -> Tensor:
     B, H, S, D = q.shape
     G = s.shape[-1]
     return (q.view(B, H, S, G, D // G).to(s.dtype) * s.unsqueeze(-1)).view(B, H, S, D)
+
+
+def _dequant(k, v, like: Tensor):
+    """fp16 [B, H, n, 128] of K and V, each (view, format, group size) or None, over the n tokens
+    of ``like`` [B, H, n, .] (kvq_dequant: one launch, rounded as the torch expressions above)."""
+    B, H, n = like.shape[:3]
+    outs = [None if x is None else torch.empty(B, H, n, 128, dtype=torch.float16, device=like.device)
+            for x in (k, v)]
+    if n:
+        args = []
+        for x, o in zip((k, v), outs):
+            args += [None, 0, 0, None] if x is None else [ctypes.byref(x[0]), x[1], x[2], o.data_ptr()]
+        C.check(C.lib().kvq_dequant(*args, B, H, n, ctypes.c_void_p(C.stream_handle(like.device))))
+    return tuple(outs)
 
 
 class _StaticG32Cache(_EngineBase):
@@ -1456,14 +1481,20 @@ class _KiviFamily(_EngineBase):
         role_aware_allocator_cache.py:402-440): code x s + z in fp32, then cast."""
         kc, vc, ks, kz, vs, vz = self.get_kivi_tensors(layer_id)
         kb, vb = self._bits[layer_id]
+        hip = self.dtype == torch.float16  # quantized sides in one HIP launch
+        if hip:
+            from .kernels import kv_view_kivi
+
+            k, v = _dequant(None if kb == 16 else (kv_view_kivi(kc, ks, kz, True), _kivi_format(kb), 32),
+                            None if vb == 16 else (kv_view_kivi(vc, vs, vz, False), _kivi_format(vb), 32), kc)
         if kb == 16:
             k = kc.to(self.dtype)
-        else:
+        elif not hip:
             kq = _unpack(kc) if kb == 4 else kc
             k = (kq.float() * ks.unsqueeze(2) + kz.unsqueeze(2)).to(self.dtype)
         if vb == 16:
             v = vc.to(self.dtype)
-        else:
+        elif not hip:
             vq = _unpack(vc) if vb == 4 else vc
             v = (vq.float() * vs.unsqueeze(-1) + vz.unsqueeze(-1)).to(self.dtype)
         rlen = self._res_len[layer_id]
@@ -2036,15 +2067,31 @@ class MixedKVCache(_EngineBase):
         in fp32, then cast."""
         kc, ks, vc, vs, vz = self.get_mixed_tensors(layer_id)
         kb, vb = self._bits[layer_id]
+        kz = self.get_k_zero_points(layer_id)
+        hip = self.dtype == torch.float16  # quantized sides in one HIP launch
+        if hip:
+            from .kernels import kv_view_kivi, kv_view_tok
+
+            def side(bits, c, s, z, gs):
+                if bits == 16:
+                    return None
+                if bits == 8:
+                    return kv_view_tok(c, s), C.KVQ_FMT_INT8_SYM, gs
+                return kv_view_kivi(c, s, z, False), C.KVQ_FMT_INT4_KIVI, 32
+
+            k, v = _dequant(side(kb, kc, ks, kz, self.k_group_size), side(vb, vc, vs, vz, self.v_group_size), kc)
         if kb == 16:
             k = kc.to(self.dtype)
+        elif hip:
+            pass
         elif kb == 8:
             k = _deq_sym(kc, ks.float()).to(self.dtype)
         else:
-            kz = self.get_k_zero_points(layer_id)
             k = (_unpack(kc).float() * ks.unsqueeze(-1) + kz.unsqueeze(-1)).to(self.dtype)
         if vb == 16:
             v = vc.to(self.dtype)
+        elif hip:
+            pass
         elif vb == 8:
             v = _deq_sym(vc, vs.float()).to(self.dtype)
         else:

@@ -19,6 +19,14 @@ int kvq_kivi_channel_range(const void* x, int64_t stride_b, int64_t stride_h, in
                            int32_t heads, int32_t tokens, int32_t bits, float q_lo, float q_hi, float* scale,
                            float* zero_point, kvq_stream_t stream);
 
+// Dequantised fp16 rows [B, H, tokens, 128] (dense) of K and V views (either NULL: left out) in
+// the formats INT8_SYM / INT4_SYM (scale views as kvq_decode_attn takes them, any strides, in
+// groups of k_group / v_group) and INT8_KIVI / INT4_KIVI (fp32 scale / zero-point per channel,
+// scale_stride_g 1, or per token, scale_stride_g 0): get_kv of the engines.
+int kvq_dequant(const kvq_kv_view* k, int32_t k_format, int32_t k_group, void* k_out, const kvq_kv_view* v,
+                int32_t v_format, int32_t v_group, void* v_out, int32_t batch, int32_t heads,
+                int32_t tokens, kvq_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
