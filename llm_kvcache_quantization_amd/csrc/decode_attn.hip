@@ -631,8 +631,8 @@ static bool static_over_bt(const kvq_kv_view& v, const kvq_decode_params* p) {
 }
 
 // Per-token scales on both sides in dense token rows (static stride-0 views too): INT8 with
-// fp16 scales or INT4_SYM with fp32 scales (the dtypes the engines store), groups of 16 or
-// more, the groups of a token contiguous.  INT8 K with groups of 16 reads two fp16 scales in
+// fp16 scales or INT4_SYM with fp32 (the dtypes the engines store) or fp16 scales (the
+// reference's function-style call), groups of 16 or more, the groups of a token contiguous.  INT8 K with groups of 16 reads two fp16 scales in
 // one 4-byte load, so its scale rows must be 4-byte aligned.
 // INT8 K with per-token fp16 scales may also pair with per-token asymmetric INT4 V in the
 // KIVI layout (the reference's MixedKVCache: K INT8 symmetric per group, V INT4 asymmetric
@@ -658,6 +658,9 @@ static bool rows16_aligned(const kvq_kv_view& v) {
   return ((uintptr_t)v.codes % 16) == 0 && v.stride_b % 16 == 0 && v.stride_h % 16 == 0;
 }
 
+static bool t4h(int fam) { return fam >= kTiledT4h && fam <= kTiledT4hg16s; }
+static bool t4h_fits(const kvq_decode_params* p, int fam);
+
 static int tok_family(const kvq_decode_params* p) {
   if (p->v.layout != KVQ_LAYOUT_ROWS) return kTiledNone;
   const bool kivi_v = p->k_format == KVQ_FMT_INT8_SYM &&
@@ -669,8 +672,9 @@ static int tok_family(const kvq_decode_params* p) {
   if (gs < 16 || vgs < 16) return kTiledNone;
   if (vgs != gs && (i4 || p->v_format != KVQ_FMT_INT8_SYM)) return kTiledNone;
   const int64_t row = i4 ? kD / 2 : kD;
-  const int dt = i4 ? KVQ_DTYPE_F32 : KVQ_DTYPE_F16;
-  const int64_t es = i4 ? 4 : 2;
+  const bool half4 = i4 && p->k.scale_dtype == KVQ_DTYPE_F16;  // INT4_SYM with fp16 scales
+  const int dt = i4 && !half4 ? KVQ_DTYPE_F32 : KVQ_DTYPE_F16;
+  const int64_t es = i4 && !half4 ? 4 : 2;
   // w: elements per aligned scale load (INT8 K with groups of 16 reads two fp16 at once)
   auto ok = [&](const kvq_kv_view& v, int g, int64_t w) {
     return v.stride_t == row && v.scale_dtype == dt && v.scale != nullptr &&
@@ -678,7 +682,7 @@ static int tok_family(const kvq_decode_params* p) {
            v.scale_stride_b % w == 0 && v.scale_stride_h % w == 0 && v.scale_stride_t % w == 0 &&
            v.scale_stride_b >= 0 && v.scale_stride_h >= 0 && v.scale_stride_t >= 0;
   };
-  const int64_t wk = (!i4 && gs == 16) ? 2 : 1;
+  const int64_t wk = ((!i4 || half4) && gs == 16) ? 2 : 1;
   if (kivi_v) {
     if (!ok(p->k, gs, wk)) return kTiledNone;
     if (p->v_format == KVQ_FMT_FP16)  // fp16 V in dense 256-byte rows
@@ -695,9 +699,15 @@ static int tok_family(const kvq_decode_params* p) {
     // gathered in LDS
     const kvq_kv_view& v = p->v;
     const int64_t ng = kD / vgs;
+    // (the scale bytes of a slab a multiple of 16 too: a load past the slab's end reads zeros)
     const bool staged = vgs <= 32 && v.scale_stride_t == ng && v.scale_stride_g == 1 &&
-                        ((uintptr_t)v.scale % 16) == 0 && (v.scale_stride_b * 4) % 16 == 0 &&
-                        (v.scale_stride_h * 4) % 16 == 0 && rows16_aligned(v);
+                        ((uintptr_t)v.scale % 16) == 0 && (v.scale_stride_b * es) % 16 == 0 &&
+                        (v.scale_stride_h * es) % 16 == 0 && (p->capacity * ng * es) % 16 == 0 &&
+                        rows16_aligned(v);
+    if (half4) {
+      const int fam = staged ? (gs == 16 ? kTiledT4hg16s : kTiledT4hs) : (gs == 16 ? kTiledT4hg16 : kTiledT4h);
+      return t4h_fits(p, fam) ? fam : (int)kTiledNone;
+    }
     if (staged) return gs == 16 ? kTiledT4g16s : kTiledT4s;
     return gs == 16 ? kTiledT4g16 : kTiledT4;
   }
@@ -751,19 +761,17 @@ static int tiled_family(const kvq_decode_params* p) {
   return tok_family(p);
 }
 
-// the split-K kernel kvq_decode_attn launches for p (nullptr if unsupported)
-static const void* kernel_for(const kvq_decode_params* p) {
-  const int fam = tiled_family(p);
+// the split-K kernel kvq_decode_attn launches for p as tiled family fam (kTiledNone: a row kernel;
+// nullptr if unsupported)
+static const void* kernel_for(const kvq_decode_params* p, int fam) {
   if (fam != kTiledNone) return tiled_kernel(fam, p->q_heads / p->kv_heads).fn;
   if (p->v.layout == KVQ_LAYOUT_TILE32) return nullptr;
   return select_kernel(family(p->k_format, p->v_format, p->k.scale_dtype == KVQ_DTYPE_F32,
                               p->v.scale_dtype == KVQ_DTYPE_F32, p->k.n_outlier > 0));
 }
 
-// waves per work-group of the split-K kernel kvq_decode_attn launches for p
-static int waves_for(const kvq_decode_params* p) {
-  return tiled_family(p) != kTiledNone ? kTiledWaves : kWaves;
-}
+// waves per work-group of that kernel
+static int waves_for(int fam) { return fam != kTiledNone ? kTiledWaves : kWaves; }
 
 // Tokens per work-group: fill every resident work-group slot exactly once when the
 // context is long enough (one wave of work-groups, no tail), in multiples of the
@@ -773,17 +781,17 @@ static int waves_for(const kvq_decode_params* p) {
 // (work-groups past a short context exit at once).  Measured on MI355X: 16 tiles per wave
 // is the best split at configs 2, 3 (uniform 32k contexts) and 4 (ragged 4k-64k).
 constexpr int kTiledMaxTiles = 16;
-int32_t choose_chunk(const kvq_decode_params* p) {
+static int32_t choose_chunk(const kvq_decode_params* p, int fam) {
   if (p->chunk_tokens > 0) return p->chunk_tokens;
   const int64_t units = (int64_t)p->batch * p->kv_heads;
-  const void* fn = kernel_for(p);
-  const int nw = waves_for(p);
+  const void* fn = kernel_for(p, fam);
+  const int nw = waves_for(fam);
   const int64_t slots = fn ? resident_slots(fn, nw * 64) : 1024;
   int64_t per_unit = slots / (units > 0 ? units : 1);
   if (per_unit < 1) per_unit = 1;
   int64_t c = (p->capacity + per_unit - 1) / per_unit;
   c = ((c + kTile * nw - 1) / (kTile * nw)) * (kTile * nw);
-  if (tiled_family(p) != kTiledNone && c > (int64_t)kTiledMaxTiles * nw * kTile)
+  if (fam != kTiledNone && c > (int64_t)kTiledMaxTiles * nw * kTile)
     c = (int64_t)kTiledMaxTiles * nw * kTile;
   if (c < kMinChunk) c = kMinChunk;
   const int64_t min_for_cap = (p->capacity + kMaxChunks - 1) / kMaxChunks;
@@ -919,15 +927,15 @@ struct Split {
   bool share;
 };
 constexpr int kShareMaxRows = 64;
-static Split plan_split(const kvq_decode_params* p) {
+static Split plan_split(const kvq_decode_params* p, int fam) {
   Split sp;
-  sp.chunk = choose_chunk(p);
+  sp.chunk = choose_chunk(p, fam);
   sp.u = sp.grid_x = sp.pitch = n_chunks_for(p, sp.chunk);
   sp.share_c = 0;
   sp.share = false;
-  if (tiled_family(p) != kTiledNone && p->context_lens != nullptr && p->chunk_tokens <= 0 &&
+  if (fam != kTiledNone && p->context_lens != nullptr && p->chunk_tokens <= 0 &&
       p->batch >= 2 && p->batch <= kShareMaxRows && p->capacity > 0 && sp.u <= kUnitChunks) {
-    const void* fn = tiled_kernel(tiled_family(p), p->q_heads / p->kv_heads).fn_share;
+    const void* fn = tiled_kernel(fam, p->q_heads / p->kv_heads).fn_share;
     const int64_t slots = fn ? resident_slots(fn, kTiledWaves * 64) : 256;
     int64_t c = slots / p->kv_heads;
     if (c < p->batch) c = p->batch;
@@ -946,20 +954,39 @@ static Split plan_split(const kvq_decode_params* p) {
   return sp;
 }
 
-}  // namespace kvq
-
-using namespace kvq;
-
-extern "C" int32_t kvq_decode_chunk_tokens(const kvq_decode_params* p) {
-  return p ? choose_chunk(p) : 0;
-}
-
 // workspace: the counter slots [B, Hkv] x 128 bytes of the tiled kernel's single-launch
 // merge (256-byte aligned size), then partial acc [B, Hq, n_chunks, 128] f32 and partial
 // (m, l) [B, Hq, n_chunks] float2.  The counters come first so that their place depends
 // only on B x Hkv: a zero-filled workspace can serve calls with other split counts.
 static int64_t counter_bytes(const kvq_decode_params* p) {
   return (((int64_t)p->batch * p->kv_heads * kCtrSlotWords * 4 + 255) / 256) * 256;
+}
+static int64_t split_bytes(const kvq_decode_params* p, const Split& sp) {
+  return counter_bytes(p) + (int64_t)p->batch * p->q_heads * sp.pitch * (kD * 4 + 8) + 256;
+}
+
+// (Row kernel and combine launch against the tiled families, us per call: 2 heads x 517 tokens 10.4
+// / 7.6, 6 ragged rows x 4 heads of up to 7999 tokens 17.8 / 14.5, 1 x 4 x 32768 in groups of 128
+// 24.3 / 13.9, 8 x 4 x 32768 55.0 / 37.7, 16 ragged rows x 8 heads of up to 4096 31.0 / 19.8.)
+// The fp16-scale INT4 families serve calls the row kernel served before them, under every limit
+// it has: slabs its 64-bit addressing covers but 32-bit buffer offsets do not, and workspaces
+// within kvq_decode_attn_noalloc's scratch where its own are (the tiled kernels' shared split may
+// keep more partials), stay with the row kernel.
+static bool t4h_fits(const kvq_decode_params* p, int fam) {
+  if (p->batch <= 0 || p->kv_heads <= 0 || p->q_heads <= 0) return false;
+  const int64_t lim = (int64_t)1 << 31, cap = p->capacity + kTile;
+  for (const int64_t row : {(int64_t)kD / 2, 2 * p->k.scale_stride_t, 2 * p->v.scale_stride_t})
+    if (row >= lim || cap >= lim || cap * row >= lim) return false;
+  return split_bytes(p, plan_split(p, fam)) <= KVQ_NOALLOC_SCRATCH_BYTES ||
+         split_bytes(p, plan_split(p, kTiledNone)) > KVQ_NOALLOC_SCRATCH_BYTES;
+}
+
+}  // namespace kvq
+
+using namespace kvq;
+
+extern "C" int32_t kvq_decode_chunk_tokens(const kvq_decode_params* p) {
+  return p ? choose_chunk(p, tiled_family(p)) : 0;
 }
 
 // the n counter slots at ctr set to zero (a fill kernel rather than a memset, so that a
@@ -979,8 +1006,7 @@ static int clear_arrival_counts(uint32_t* ctr, int64_t n, hipStream_t s) {
 
 extern "C" int64_t kvq_decode_workspace_bytes(const kvq_decode_params* p) {
   if (!p) return 0;
-  const int64_t rows = (int64_t)p->batch * p->q_heads * plan_split(p).pitch;
-  return counter_bytes(p) + rows * (kD * 4 + 8) + 256;
+  return split_bytes(p, plan_split(p, tiled_family(p)));
 }
 
 // kvq_decode_attn, and with app != nullptr kvq_append_decode_attn (tiled path only; the
@@ -1048,13 +1074,14 @@ static int decode_impl(const kvq_decode_params* p, const FusedAppend* app, kvq_s
     return fail(KVQ_ERR_UNSUPPORTED, "a V group size apart from K's needs per-token INT8 V on the "
                                      "tiled kernel (dense rows, groups of 16 or more)");
 
-  const Split sp = plan_split(p);
+  // (the split the caller sized the workspace for)
+  const Split sp = plan_split(p, fam_override >= 0 ? tiled_family(p) : tfam);
   const int32_t chunk = sp.chunk;
   if (chunk <= 0 || chunk % kTile)
     return fail(KVQ_ERR_INVALID, "chunk_tokens must be a positive multiple of 32");
   const int64_t nch64 = sp.pitch;
   if (nch64 > kMaxChunks) return fail(KVQ_ERR_UNSUPPORTED, "too many chunks (raise chunk_tokens)");
-  const int64_t need = kvq_decode_workspace_bytes(p);
+  const int64_t need = split_bytes(p, sp);
   if (!p->workspace || p->workspace_bytes < need)
     return fail(KVQ_ERR_INVALID, "workspace too small: need " + std::to_string(need) + " bytes");
   if (!aligned(p->workspace, 16)) return fail(KVQ_ERR_INVALID, "workspace must be 16-byte aligned");
@@ -1076,7 +1103,7 @@ static int decode_impl(const kvq_decode_params* p, const FusedAppend* app, kvq_s
   a.u_chunks = (int)sp.u;
   a.share_c = (int)sp.share_c;
   a.strided = tiled ? 1 : 0;
-  a.nw = waves_for(p);
+  a.nw = waves_for(tfam);
   const int64_t rows = (int64_t)p->batch * p->q_heads * nch64;
   char* ws = reinterpret_cast<char*>(p->workspace);
   a.counters = reinterpret_cast<uint32_t*>(ws);
@@ -1322,6 +1349,7 @@ extern "C" int kvq_append_decode_attn(const kvq_decode_params* p, const kvq_appe
                                       const kvq_append_params* v_new, kvq_stream_t stream) {
   if (!p) return fail(KVQ_ERR_INVALID, "params is NULL");
   int fam = tiled_family(p);
+  if (t4h(fam)) fam = kTiledNone;  // (fp16-scale INT4: attention only)
   bool spec = fam == kTiledA4A4 || fam == kTiledA4A4o || fam == kTiledI8A4 ||
               fam == kTiledI8I8 || fam == kTiledI8I8g;
   // per-token scale views of one row and one token look static to tiled_family; an append

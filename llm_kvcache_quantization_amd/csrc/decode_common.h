@@ -462,6 +462,8 @@ enum TiledFam {
   // kTiledKivi / kTiledT8Kv / kTiledT8Kvg16 with 16-byte aligned V code rows: the V rows read
   // with 16-byte loads and gathered through LDS (VKiviRowTS)
   kTiledKivis, kTiledT8Kvs, kTiledT8Kvg16s,
+  // the kTiledT4 families with fp16 scales (no fused append)
+  kTiledT4h, kTiledT4hg16, kTiledT4hs, kTiledT4hg16s,
 };
 // a tiled kernel and the formats of the fused row append built into it (-1: none)
 struct TiledFn {
@@ -472,6 +474,7 @@ struct TiledFn {
 // the instantiations, one lookup per translation unit (fn nullptr: not one of its families)
 TiledFn tiled_kernel_a4(int fam, bool pack8);
 TiledFn tiled_kernel_tok(int fam, bool pack8);
+TiledFn tiled_kernel_t4h(int fam, bool pack8);
 TiledFn tiled_kernel_kv4(int fam, bool pack8);
 TiledFn tiled_kernel_kv16(int fam, bool pack8);
 TiledFn tiled_kernel_kt(int fam, bool pack8);

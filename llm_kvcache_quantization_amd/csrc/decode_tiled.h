@@ -1665,8 +1665,11 @@ __device__ __forceinline__ uint32_t scale_bytes(int64_t cap, int64_t sst, int gs
   return (uint32_t)(sst > 0 ? cap * sst * es : (int64_t)(kD / gs) * es);
 }
 
-template <bool I4, int NS>
+// SH (INT4 only): fp16 scales, as the reference's function-style call takes them
+// (src/kernels/triton_decode_attn_int4.py:62-121); no fused append (the engines store fp32).
+template <bool I4, int NS, bool SH = false>
 struct KTokT {
+  static constexpr bool kF32S = I4 && !SH;  // fp32 scales
   static constexpr int kRowFmt = I4 ? KVQ_FMT_INT4_SYM : KVQ_FMT_INT8_SYM;  // the fused append's K format
   static_assert(NS == 1 || NS == 2, "groups of 16 or more");
   // (16 cost the per-token INT8 / INT4 baselines 0.35 / 0.6 us per launch at config 3's
@@ -1677,14 +1680,15 @@ struct KTokT {
   static constexpr bool kAppend = false;
   // the writer runs quant_row_x (fused step); with INT4_SYM sides it also finds the group
   // rescue's threshold over every row of the append (rescue_thr_wave)
-  static constexpr bool kAppendRow = true;
+  static constexpr bool kAppendRow = !SH;
   static constexpr bool kRescue = I4;
+  static constexpr bool kRowArgs = true;  // the prologue reads most argument lines
   static constexpr bool kAsym = false;
   static constexpr bool kGsAny = true;
   static constexpr bool kOut = false;
   static constexpr bool kSub24 = false;  // logits at unit scale
   static constexpr int kRow = I4 ? kD / 2 : kD;  // code bytes per token
-  static constexpr int kEs = I4 ? 4 : 2;         // scale bytes (fp32 / fp16)
+  static constexpr int kEs = kF32S ? 4 : 2;      // scale bytes (fp32 / fp16)
   half8v qh[4];
   rsrc_t rk, rs;
   uint32_t vk, vs, sst;  // lane code offset, lane scale offset, scale bytes per token
@@ -1692,7 +1696,7 @@ struct KTokT {
     u32x4 w[I4 ? 2 : 4];  // I4: [rb] = bytes [16 lg, 16 lg + 16) of token 16 rb + row;
                           // INT8: [2 rb + i] = bytes [32 lg + 16 i, + 16)
     uint32_t s[2];        // the NS scales of row block rb (fp16 pair, fp16 or fp32 bits)
-    uint32_t s2[I4 && NS == 2 ? 2 : 1];  // the second fp32 scale of row block rb (NS = 2)
+    uint32_t s2[kF32S && NS == 2 ? 2 : 1];  // the second fp32 scale of row block rb (NS = 2)
   };
 
   __device__ void setup_addr(const DecodeArgs& a, int b, int hkv, int lane) {
@@ -1753,12 +1757,12 @@ struct KTokT {
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       const uint32_t o = p + (uint32_t)rb * 16u * sst;
-      if constexpr (I4 && NS == 2) {
+      if constexpr (kF32S && NS == 2) {
         const u32x2 s = __builtin_bit_cast(
             u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, (int)o, 0, kBufNT));
         r.s[rb] = s.x;
         r.s2[rb] = s.y;
-      } else if constexpr (I4 || NS == 2) {
+      } else if constexpr (kF32S || NS == 2) {
         r.s[rb] = bload1(rs, o, 0);  // one fp32, or two fp16
       } else {
         r.s[rb] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rs, (int)o, 0, kBufNT);
@@ -1768,7 +1772,7 @@ struct KTokT {
   // the fp16 scale of slice j in row block rb, twice
   __device__ __forceinline__ uint32_t scale2(const Raw& r, int rb, int j) const {
     half_t s;
-    if constexpr (I4) {
+    if constexpr (kF32S) {
       const uint32_t bits = (NS == 2 && j >= 2) ? r.s2[rb] : r.s[rb];
       s = (half_t)__builtin_bit_cast(float, bits);
     } else {
@@ -1817,8 +1821,10 @@ struct KTokT {
 // passed through the wave's own LDS (stage()), from which each lane reads its gathered
 // operands with ds_read2_b32; the same operands reach the MFMAs as with the 8 + 8 dword
 // gathers per lane and tile that the other instantiation issues.
-template <bool I4, bool STAGE = false>
+// SH (INT4 only): fp16 scales.
+template <bool I4, bool STAGE = false, bool SH = false>
 struct VTokT {
+  static constexpr bool kF32S = I4 && !SH;  // fp32 scales
   static constexpr bool kStage = I4 && STAGE;
   // LDS layout of a staged tile (per wave): the 32 code rows (Rows64Lds), then the 32 scale
   // rows (16 or 32 bytes: groups of 32 or 16), 48 bytes apart (so that the 4 rows one read
@@ -1831,7 +1837,7 @@ struct VTokT {
   static constexpr bool kPackedPV = false;
   static constexpr bool kTile32 = false;
   static constexpr int kRow = I4 ? kD / 2 : kD;
-  static constexpr int kEs = I4 ? 4 : 2;
+  static constexpr int kEs = kF32S ? 4 : 2;
   __device__ __forceinline__ void finalize(float4v*, int) const {}
   __device__ __forceinline__ float* extra() { return nullptr; }
   rsrc_t rv, rs;
@@ -1839,7 +1845,7 @@ struct VTokT {
   // kStage: the code rows' staging, the lane's scale-block load offset, LDS write offset and
   // read base
   Rows64Lds cst;
-  uint32_t ls, ws, rsb;
+  uint32_t ls, ws, ws2, rsb;
   struct Raw {
     uint32_t w[8][I4 ? 1 : 2];  // token T(k)
     uint32_t s[8];              // token T(k)'s scale (fp32 or fp16 bits)
@@ -1866,13 +1872,15 @@ struct VTokT {
     rs = buffer_rsrc(sb, scale_bytes(a.cap, a.v.sst, a.vgs, kEs));
     vs = (uint32_t)((4 * lg) * sst + gi * a.v.ssg * kEs);
     if constexpr (kStage) {
-      // a token's scale row: sst = 4 * (128 / gs) bytes, 32 (groups of 16) or 16 (of 32)
+      // a token's scale row: sst = kEs * (128 / gs) bytes, 32 / 16 (fp32 / fp16, groups of 16) or
+      // 16 / 8 (of 32; a lane's 16 bytes then hold two rows)
       const uint32_t byte = (uint32_t)lane * 16u;
       cst.setup(lane);
       ls = byte < 32u * sst ? byte : kOutOfRange;
       ws = kSOff + (byte / sst) * kSRow + byte % sst;
+      ws2 = kSOff + ((byte + 8u) / sst) * kSRow + (byte + 8u) % sst;
       // pair p reads the scales of tokens T(2 p), T(2 p) + 1 = 4 lg + {0, 2, 16, 18}[p] + {0, 1}
-      rsb = kSOff + (uint32_t)(4 * lg) * kSRow + (uint32_t)gi * 4u;
+      rsb = kSOff + (uint32_t)(4 * lg) * kSRow + (uint32_t)gi * kEs;
     }
   }
   // kStage: write the tile's rows and scales to the wave's LDS and read back the lane's
@@ -1882,7 +1890,14 @@ struct VTokT {
       __shared__ __attribute__((aligned(16))) uint8_t vst[kTW][kStageBytes];
       uint8_t* base = vst[wave];
       cst.write(base, r.c0, r.c1);
-      if (ls != kOutOfRange) *reinterpret_cast<u32x4*>(base + ws) = r.sc;
+      if (ls != kOutOfRange) {
+        if constexpr (kF32S) {
+          *reinterpret_cast<u32x4*>(base + ws) = r.sc;
+        } else {
+          *reinterpret_cast<u32x2*>(base + ws) = u32x2{r.sc.x, r.sc.y};
+          *reinterpret_cast<u32x2*>(base + ws2) = u32x2{r.sc.z, r.sc.w};
+        }
+      }
       uint32_t w[8];
       cst.gather(base, w);
 #pragma unroll
@@ -1890,9 +1905,15 @@ struct VTokT {
         const uint32_t dt = p == 0 ? 0u : p == 1 ? 2u : p == 2 ? 16u : 18u;
         r.w[2 * p][0] = w[2 * p];
         r.w[2 * p + 1][0] = w[2 * p + 1];
-        const uint32_t* sr = reinterpret_cast<const uint32_t*>(base + rsb + dt * kSRow);
-        r.s[2 * p] = sr[0];
-        r.s[2 * p + 1] = sr[kSRow / 4];
+        if constexpr (kF32S) {
+          const uint32_t* sr = reinterpret_cast<const uint32_t*>(base + rsb + dt * kSRow);
+          r.s[2 * p] = sr[0];
+          r.s[2 * p + 1] = sr[kSRow / 4];
+        } else {
+          const uint16_t* sr = reinterpret_cast<const uint16_t*>(base + rsb + dt * kSRow);
+          r.s[2 * p] = sr[0];
+          r.s[2 * p + 1] = sr[kSRow / 2];
+        }
       }
     } else {
       (void)r;
@@ -1913,7 +1934,8 @@ struct VTokT {
       const uint32_t t = (k < 4) ? (uint32_t)k : (uint32_t)(12 + k);  // 16 + k - 4
       if constexpr (I4) {
         r.w[k][0] = bload1(rv, v + t * kRow, 0);
-        r.s[k] = bload1(rs, p + t * sst, 0);
+        r.s[k] = kF32S ? bload1(rs, p + t * sst, 0)
+                       : (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rs, (int)(p + t * sst), 0, kBufNT);
       } else {
         const u32x2 x = __builtin_bit_cast(
             u32x2, __builtin_amdgcn_raw_buffer_load_b64(rv, (int)(v + t * kRow), 0, kBufNT));
@@ -1933,7 +1955,7 @@ struct VTokT {
     }
   }
   __device__ __forceinline__ uint32_t spair(const Raw& r, int p) const {
-    if constexpr (I4)
+    if constexpr (kF32S)
       return pair_h2((half_t)__builtin_bit_cast(float, r.s[2 * p]),
                      (half_t)__builtin_bit_cast(float, r.s[2 * p + 1]));
     else
@@ -2286,6 +2308,12 @@ struct v_staged : std::false_type {};
 template <class T>
 struct v_staged<T, std::void_t<decltype(T::kStage)>> : std::bool_constant<T::kStage> {};
 
+// K operand types whose prologue reads most argument lines without a fused append
+template <class T, class = void>
+struct row_args : std::bool_constant<T::kAppendRow> {};
+template <class T>
+struct row_args<T, std::void_t<decltype(T::kRowArgs)>> : std::true_type {};
+
 template <class KF, class VF, int LOOK, bool PACK8, bool SHARE, int WPE = 2>
 __global__ __launch_bounds__(kTW * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void decode_tiled_kernel(DecodeArgs a) {
@@ -2300,7 +2328,7 @@ void decode_tiled_kernel(DecodeArgs a) {
   // them (touching their lines in every wave cost the shared split 0.27 us per launch); the
   // shared split of the other formats touches the lines before the append's and the
   // append's first (0.15 us per launch against every line up to the row sides).
-  if constexpr (KF::kAppendRow) {
+  if constexpr (row_args<KF>::value) {
     const uint32_t* w = reinterpret_cast<const uint32_t*>(&a);
 #pragma unroll
     for (int i = 0; i < (int)(__builtin_offsetof(DecodeArgs, ark) / 4); i += 16)
