@@ -40,6 +40,7 @@ for them.
 from __future__ import annotations
 
 import ctypes
+import functools
 import logging
 import math
 import os
@@ -111,9 +112,13 @@ class _EngineBase:
         self._layer_capacity: List[int] = [0] * num_layers
         self._seq_len = 0
         self.decode_stats: Dict[str, object] = _new_decode_stats()
+        # status words: counters that the host reads as differences to what it saw last, so that
+        # no launch clears them (cleared after a NaN / Inf flag)
         self._status: Optional[Tensor] = None
+        self._status_seen: List[int] = [0] * 4
         # the decode step's per-layer status rows and the appends not read yet
         self._step_status: Optional[Tensor] = None
+        self._step_seen: List[List[int]] = []
         self._step_pending: List[tuple] = []
         self._step_seq_len0 = 0
         # per layer: the LayerStep over the layer's buffers and the fused append's parameter
@@ -179,7 +184,8 @@ class _EngineBase:
             raise ValueError(f"v must be 4D [B,H,S,D], got ndim={v.ndim}")
         if k.shape != v.shape:
             raise ValueError(f"k/v shape mismatch: k={tuple(k.shape)} vs v={tuple(v.shape)}")
-        if k.device.type != self._dev_type or v.device.type != self._dev_type:
+        if not (k.is_cuda and v.is_cuda and self._dev_type == "cuda") and (
+                k.device.type != self._dev_type or v.device.type != self._dev_type):
             raise ValueError(
                 f"Device mismatch: cache_device={torch.device(self.device)}, k.device={k.device}, "
                 f"v.device={v.device}")
@@ -195,6 +201,7 @@ class _EngineBase:
     def _status_buf(self, device) -> Tensor:
         if self._status is None or self._status.device != device:
             self._status = torch.zeros(4, dtype=torch.int32, device=device)
+            self._status_seen = [0] * 4
         return self._status
 
     # -- the decode step's status words, read once per step.  ``append`` checks its input
@@ -213,6 +220,7 @@ class _EngineBase:
             self._flush_step_status()
             buf = self._step_status = torch.zeros(self.num_layers, 4, dtype=torch.int32,
                                                   device=device)
+            self._step_seen = [[0] * 4 for _ in range(self.num_layers)]
         elif any(e[0] == layer_id for e in self._step_pending):
             self._flush_step_status()
         if not self._step_pending:  # the first append of a step: its length before the step
@@ -238,32 +246,39 @@ class _EngineBase:
         if not pending:
             return
         self._step_pending = []
-        rows = self._step_status.cpu()
-        self._step_status.zero_()
+        rows, seen = self._step_status.cpu().tolist(), self._step_seen
+        self._step_seen = rows
         bad = None
         for layer_id, n_elem, kind, qrange, clip_warn in pending:
-            st = rows[layer_id].tolist()
+            st = _since(rows[layer_id], seen[layer_id])
             if bad is None and (st[0] & 1 or st[2] & 1):
                 bad = (kind, "K" if st[0] & 1 else "V")
             if clip_warn:
                 self._clip_warnings(layer_id, n_elem, qrange, st)
         if bad is not None:
+            self._discard_step_status(True)
             for layer_id, *_ in pending:
                 self._layer_seq_lens[layer_id] -= 1
             self._seq_len = self._step_seq_len0
             raise ValueError(f"{bad[0]} append: {bad[1]} input contains NaN or Inf — refusing "
                              "to quantize corrupt data")
 
-    def _discard_step_status(self) -> None:
-        self._step_pending = []
-        if self._step_status is not None:
+    def _discard_step_status(self, unread: bool = False) -> None:
+        """Drops the pending rows; clears the buffer if it holds counts not read (or `unread`)."""
+        if (self._step_pending or unread) and self._step_status is not None:
             self._step_status.zero_()
+            self._step_seen = [[0] * 4 for _ in range(self.num_layers)]
+        self._step_pending = []
 
     def _read_status(self) -> List[int]:
-        """The append kernel's status words (NaN flags and clip counts of K and V), then
-        cleared for the next append."""
-        st = self._status.cpu().tolist()
-        self._status.zero_()
+        """The append kernel's status words (NaN flags and clip counts of K and V) since the
+        last read."""
+        now = self._status.cpu().tolist()
+        st = _since(now, self._status_seen)
+        if st[0] or st[2]:
+            self._status.zero_()
+            now = [0] * 4
+        self._status_seen = now
         return st
 
     def _check_status(self, layer_id: int, n_elem: int, kind: str, qrange: str) -> None:
@@ -287,6 +302,13 @@ class _EngineBase:
     def _launch_append(self, pk: C.AppendParams, pv: C.AppendParams, device) -> None:
         C.check(C.lib().kvq_quant_append(ctypes.byref(pk), ctypes.byref(pv),
                                          ctypes.c_void_p(C.stream_handle(device))))
+
+
+def _since(now: List[int], seen: List[int]) -> List[int]:
+    """Status words [K flags, K count, V flags, V count] read now, less what was seen before: the
+    counts as 32-bit differences (the counters may wrap), the flags as they are (they are cleared
+    when one is set)."""
+    return [now[0], (now[1] - seen[1]) & 0xFFFFFFFF, now[2], (now[3] - seen[3]) & 0xFFFFFFFF]
 
 
 def _dyn_quantile(percentile: float) -> float:
@@ -313,6 +335,16 @@ def _fill_append(p: C.AppendParams, fmt: int, x: Tensor, gs: int, codes: Tensor,
     p.write_pos = write_pos
     p.capacity = codes.shape[2]
     p.status = status_ptr
+
+
+def _set_rows(p: C.AppendParams, x: Tensor) -> None:
+    """The new rows' address and strides in a kept parameter block (strides as last time are not
+    set again)."""
+    p.x = x.data_ptr()
+    strides = x.stride()
+    if strides != getattr(p, "_strides", None):
+        p.x_stride_b, p.x_stride_h, p.x_stride_s = strides[:3]
+        p._strides = strides
 
 
 class _SymCacheBase(_EngineBase):
@@ -365,6 +397,15 @@ class _SymCacheBase(_EngineBase):
         pass
 
     def _ensure_capacity(self, layer_id, batch, heads, head_dim, num_groups, target_len):
+        # (what the full checks below accept without growing, as a decode step finds it)
+        if target_len <= self._layer_capacity[layer_id]:
+            kb, ks = self._k_cache[layer_id], self._k_scale[layer_id]
+            if kb is not None and ks is not None and self._v_cache[layer_id] is not None \
+                    and self._v_scale[layer_id] is not None:
+                shape = kb.shape
+                if shape[0] == batch and shape[1] == heads and shape[3] == self._code_dim(head_dim) \
+                        and ks.shape[-1] == num_groups:
+                    return
         bufs = [self._k_cache[layer_id], self._v_cache[layer_id],
                 self._k_scale[layer_id], self._v_scale[layer_id]]
         non_none = sum(b is not None for b in bufs)
@@ -534,8 +575,7 @@ class _SymCacheBase(_EngineBase):
         for p, x, off in ((pk, k, 0), (pv, v, 8)):
             if x.stride(-1) != 1:
                 x = x.contiguous()
-            p.x = x.data_ptr()
-            p.x_stride_b, p.x_stride_h, p.x_stride_s = x.stride()[:3]
+            _set_rows(p, x)
             p.write_pos = pos
             p.status = None if sptr is None else sptr + off
             p._keep = (x,) + p._keep_fixed
@@ -813,12 +853,8 @@ class INT4KVCache(_SymCacheBase):
             return True
         if B is None or H is None:
             return False
-        import numpy as np
-
         n = B * H * (D // self.group_size)
-        q = np.float32(max(0.0, min(1.0, 1.0 - self.outlier_rescue_ratio)))
-        lo = int(np.floor(q * np.float32(n - 1)))
-        return B * H <= 32 and n - 1 - lo < 32
+        return B * H <= 32 and n - 1 - _rescue_rank(self.outlier_rescue_ratio, n) < 32
 
     def _policy(self, p, side):
         adaptive = self.adaptive_static_scales and (
@@ -874,6 +910,15 @@ class INT4KVCache(_SymCacheBase):
     def __repr__(self) -> str:
         return (f"INT4KVCache(num_layers={self.num_layers}, seq_len={self._seq_len}, "
                 f"memory={self.get_memory_mb():.2f}MB)")
+
+
+@functools.lru_cache(maxsize=256)
+def _rescue_rank(ratio: float, n: int) -> int:
+    """The lower rank of torch.quantile at 1 - ratio over n scales (fp32, as the kernels compute it)."""
+    import numpy as np
+
+    q = np.float32(max(0.0, min(1.0, 1.0 - ratio)))
+    return int(np.floor(q * np.float32(n - 1)))
 
 
 def _unpack(packed: Tensor) -> Tensor:
@@ -1106,8 +1151,7 @@ class _StaticG32Cache(_EngineBase):
         for p, x, off in ((pk, k, 0), (pv, v, 8)):
             if x.stride(-1) != 1:
                 x = x.contiguous()
-            p.x = x.data_ptr()
-            p.x_stride_b, p.x_stride_h, p.x_stride_s = x.stride()[:3]
+            _set_rows(p, x)
             p.write_pos = old
             p.status = None if sptr is None else sptr + off
             p._keep = (x,)
@@ -1634,8 +1678,7 @@ class _KiviFamily(_EngineBase):
         for p, x in ((pk, k), (pv, v)):
             if x.stride(-1) != 1:
                 x = x.contiguous()
-            p.x = x.data_ptr()
-            p.x_stride_b, p.x_stride_h, p.x_stride_s = x.stride()[:3]
+            _set_rows(p, x)
             p.write_pos = pos
             p._keep = (x,)
         return pk, pv

@@ -153,7 +153,7 @@ def _shared_workspace(device, nbytes: int, units: int) -> torch.Tensor:
     call leaves zero, and the partials follow them: calls with the same units ordered on
     one stream can share it.  Another units count or stream gets its own (a larger count
     would find its counters where partials were written)."""
-    key = (str(device), torch.cuda.current_stream(device).cuda_stream, int(units))
+    key = (device, C.stream_handle(device), units)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
@@ -226,9 +226,13 @@ class DecodePlan:
         p.out = self.out.data_ptr()
         p.out_stride_b, p.out_stride_h = self.out.stride(0), self.out.stride(1)
         self.params = p
-        self.chunk_tokens = int(L.kvq_decode_chunk_tokens(ctypes.byref(p)))
-        self._pp = ctypes.byref(self.params)
+        self._pp = ctypes.byref(p)
         self.device = q.device
+
+    @property
+    def chunk_tokens(self) -> int:
+        """Tokens per work-group of the plan's split."""
+        return int(C.lib().kvq_decode_chunk_tokens(self._pp))
 
     def launch(self, stream: Optional[int] = None) -> torch.Tensor:
         s = C.stream_handle(self.device) if stream is None else stream
@@ -286,6 +290,7 @@ class LayerStep:
             self.device = torch.device(self.device.type, torch.cuda.current_device())
         self.workspace: Optional[torch.Tensor] = None
         self._tau = None
+        self._q_strides = self._o_strides = None  # those set in the block
         # the workspace a call needs depends on the context length only through its 32-token
         # tile count (chunk sizes are multiples of 32 tokens): asked again when that changes
         self._ws_tiles = -1
@@ -294,11 +299,13 @@ class LayerStep:
                  inv_tau: Optional[torch.Tensor]) -> torch.Tensor:
         p = self.params
         p.q = q.data_ptr()
-        p.q_stride_b, p.q_stride_h = q.stride(0), q.stride(1)
-        p.inv_tau = _ptr(inv_tau)
+        strides = q.stride()
+        if strides != self._q_strides:
+            p.q_stride_b, p.q_stride_h = strides[:2]
+            self._q_strides = strides
+        p.inv_tau = None if inv_tau is None else inv_tau.data_ptr()
         self._tau = inv_tau
-        p.capacity = n
-        p.context_len = n
+        p.capacity = p.context_len = n
         p.sm_scale = float(sm_scale)
         tiles = (n + 31) >> 5
         if tiles != self._ws_tiles:
@@ -312,7 +319,10 @@ class LayerStep:
             self._ws_tiles = tiles
         out = torch.empty_like(q)
         p.out = out.data_ptr()
-        p.out_stride_b, p.out_stride_h = out.stride(0), out.stride(1)
+        strides = out.stride()
+        if strides != self._o_strides:
+            p.out_stride_b, p.out_stride_h = strides[:2]
+            self._o_strides = strides
         return out
 
     def set_residual(self, res_k: Optional[torch.Tensor], res_v: Optional[torch.Tensor], n: int) -> None:
@@ -520,9 +530,12 @@ def _decode_tok(q, k_cache, v_cache, k_scale, v_scale, context_lens, sm_scale, d
         raise ValueError(f"head_dim {hd} must be divisible by num_groups {num_groups}")
     group_size = hd // num_groups
     max_seq = int(k_cache.shape[2])
-    # the reference validates context lengths on the host (one sync); so does this wrapper
-    max_ctx = int(context_lens.max().item()) if context_lens.numel() else 0
-    min_ctx = int(context_lens.min().item()) if context_lens.numel() else 0
+    # the reference validates context lengths on the host; so does this wrapper, from one copy
+    # (a maximum and a minimum read back one by one took two reductions and two waits, 34 us
+    # against 13)
+    lens = context_lens.tolist()
+    max_ctx = int(max(lens)) if lens else 0
+    min_ctx = int(min(lens)) if lens else 0
     if min_ctx < 0:
         raise ValueError(f"context_lens must be >= 0, got min={min_ctx}")
     if max_ctx > max_seq:
