@@ -96,6 +96,40 @@ __device__ __forceinline__ int group_sum(int v, int gs) {
   return v;
 }
 
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_max_u(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a),
+                                                                __builtin_bit_cast(u16x2, b)));
+}
+
+// The two largest values (with multiplicity) of the lane's group, by DPP within rows of 16 lanes
+// and readlane between them: no trip through the LDS crossbar, whose latency made the walk below
+// the longest part of a decode step's append.  Finite values.  (Fused step of 1 x 2 kv heads x 500
+// tokens, 99.9 percentile: int8 13.2 -> 10.1 us, int4 11.8 -> 9.2, mixed 11.4 -> 9.5, with the row's
+// address and group taken without divisions; the attention alone is 8.5, 7.2 and 8.1.)
+__device__ __forceinline__ void group_top2(float a0, float a1, int gs, int lane, float& m1, float& m2) {
+#pragma clang fp contract(off)
+  m1 = fmaxf(a0, a1);
+  m2 = fminf(a0, a1);
+  auto merge = [&](float n1, float n2) {
+    m2 = fmaxf(fminf(m1, n1), fmaxf(m2, n2));
+    m1 = fmaxf(m1, n1);
+  };
+  merge(dppf<0xB1>(m1), dppf<0xB1>(m2));                    // quad_perm [1, 0, 3, 2]
+  merge(dppf<0x4E>(m1), dppf<0x4E>(m2));                    // quad_perm [2, 3, 0, 1]
+  if (gs >= 16) merge(dppf<0x141>(m1), dppf<0x141>(m2));    // row_half_mirror
+  if (gs >= 32) merge(dppf<0x140>(m1), dppf<0x140>(m2));    // row_mirror
+  if (gs >= 64) {
+    const bool upper = lane >= 32;
+    const float a1r = row_lane(m1, 0), b1r = row_lane(m1, 16), c1r = row_lane(m1, 32), d1r = row_lane(m1, 48);
+    const float a2r = row_lane(m2, 0), b2r = row_lane(m2, 16), c2r = row_lane(m2, 32), d2r = row_lane(m2, 48);
+    m1 = upper ? c1r : a1r;
+    m2 = upper ? c2r : a2r;
+    merge(upper ? d1r : b1r, upper ? d2r : b2r);
+    if (gs >= 128) merge(upper ? row_lane(m1, 0) : row_lane(m1, 32), upper ? row_lane(m2, 0) : row_lane(m2, 32));
+  }
+}
+
 // The order statistics v[lo] <= v[hi] (ascending ranks, ties broken by channel index) of
 // the gs finite values of the lane's group (a0, a1 = the lane's two values, any sign).  Near
 // the top (the reference's 99.9 percentile over groups of up to 128 takes the two largest
@@ -103,10 +137,22 @@ __device__ __forceinline__ int group_sum(int v, int gs) {
 // multiplicity c holds the ranks [gs - above - c, gs - above), `above` counting the values
 // already passed, and gs - lo steps reach rank lo.  Near the bottom the same walk runs on
 // the negated values (v[r] = -(-v)[gs - 1 - r]).  Elsewhere every value's rank is counted.
-// The group's lanes all return the results.
-__device__ inline void group_order_stats(float a0, float a1, int gs, int lo, int hi, int lane,
+// The group's lanes all return the results.  finite: every value of the wave is (else ranks within
+// the two largest or smallest take the walk too, which passes NaN and Inf by).
+__device__ inline void group_order_stats(float a0, float a1, int gs, int lo, int hi, int lane, bool finite,
                                   float& vlo, float& vhi) {
 #pragma clang fp contract(off)
+  if (finite && (lo >= gs - 2 || hi <= 1)) {
+    const float sg = lo >= gs - 2 ? 1.0f : -1.0f;
+    float m1, m2;
+    group_top2(sg * a0, sg * a1, gs, lane, m1, m2);
+    m1 *= sg;
+    m2 *= sg;
+    const int first = lo >= gs - 2 ? gs - 1 : 0;  // the rank m1 holds
+    vlo = lo == first ? m1 : m2;
+    vhi = hi == first ? m1 : m2;
+    return;
+  }
   const bool top = gs - 1 - lo < 4, bottom = !top && hi < 4;
   if (top || bottom) {
     const float sg = top ? 1.0f : -1.0f;  // bottom: walk -v from its top
@@ -145,12 +191,12 @@ __device__ inline void group_order_stats(float a0, float a1, int gs, int lo, int
 
 // torch.quantile(v, q) over the gs values of the lane's group (linear interpolation in fp32:
 // rank = fp32(q) * (gs - 1), w = rank - floor(rank))
-__device__ inline float group_quantile(float a0, float a1, int gs, float q, int lane) {
+__device__ inline float group_quantile(float a0, float a1, int gs, float q, int lane, bool finite) {
 #pragma clang fp contract(off)
   const float rank = q * (float)(gs - 1);
   const int lo = (int)floorf(rank), hi = (int)ceilf(rank);
   float vlo, vhi;
-  group_order_stats(a0, a1, gs, lo, hi, lane, vlo, vhi);
+  group_order_stats(a0, a1, gs, lo, hi, lane, finite, vlo, vhi);
   return quantile_lerp(vlo, vhi, rank - (float)lo);
 }
 
@@ -163,8 +209,10 @@ __device__ __forceinline__ float group_absmax(float v, int gs) {
   if (gs >= 8) v = fmaxf(v, dppf<0x4E>(v));          // quad_perm [2, 3, 0, 1]
   if (gs >= 16) v = fmaxf(v, dppf<0x141>(v));        // row_half_mirror
   if (gs >= 32) v = fmaxf(v, dppf<0x140>(v));        // row_mirror
-  if (gs >= 64) v = fmaxf(v, __shfl_xor(v, 16, 64));
-  if (gs >= 128) v = fmaxf(v, __shfl_xor(v, 32, 64));
+  if (gs >= 64) {  // the row maxima by readlane
+    const float lo = fmaxf(row_lane(v, 0), row_lane(v, 16)), hi = fmaxf(row_lane(v, 32), row_lane(v, 48));
+    v = gs >= 128 ? fmaxf(lo, hi) : (__lane_id() >= 32 ? hi : lo);
+  }
   return v;
 }
 
@@ -210,27 +258,35 @@ __device__ __forceinline__ half_t int8_scale16(const AppendDev& a, float stv, fl
   return (half_t)fmaxf(s, 1e-5f);                              // int8_basic.py:159
 }
 
+// the group of the lane's two channels (gs is a power of two, 8..128: a shift, where a division
+// by a value the compiler does not know is some 30 instructions)
+__device__ __forceinline__ int lane_group(const AppendDev& a, int lane) {
+  return (2 * lane) >> (31 - __builtin_clz(a.gs));
+}
+
 // the lane's two input values of append row `row` (row = (b * H + h) * S + s)
-__device__ __forceinline__ const half_t* row_x(const AppendDev& a, int row) {
-#pragma clang fp contract(off)
-  const int s_idx = row % a.S, bh = row / a.S, h = bh % a.H, b = bh / a.H;
+__device__ __forceinline__ const half_t* row_x_at(const AppendDev& a, int b, int h, int s_idx) {
   return a.x + (int64_t)b * a.xsb + (int64_t)h * a.xsh + (int64_t)s_idx * a.xss;
+}
+__device__ __forceinline__ const half_t* row_x(const AppendDev& a, int row) {
+  const int s_idx = row % a.S, bh = row / a.S;
+  return row_x_at(a, bh / a.H, bh % a.H, s_idx);
 }
 __device__ __forceinline__ half2v load_x(const AppendDev& a, int row, int lane) {
 #pragma clang fp contract(off)
   return *reinterpret_cast<const half2v*>(row_x(a, row) + 2 * lane);
 }
 
-// The static scale of the lane's group in append row `row` as its raw bits (fp32, or fp16 in
+// The static scale of the lane's group in a row of head h as its raw bits (fp32, or fp16 in
 // the low half; 0 without a static table), and their value.  The fused step's writer requests
 // the bits at the start of the kernel and converts them where it quantizes: converting at the
 // load (one branch per table dtype) made the compiler wait for every outstanding load there,
 // the q loads and the first cache tiles included.
-__device__ __forceinline__ uint32_t row_static_bits(const AppendDev& a, int row, int lane) {
+__device__ __forceinline__ uint32_t row_static_bits(const AppendDev& a, int h, int lane) {
   if (a.st == nullptr || a.fmt == KVQ_FMT_INT4_ASYM || a.fmt == KVQ_FMT_INT4_KIVI ||
       a.fmt == KVQ_FMT_INT8_KIVI)
     return 0u;
-  const int64_t off = (int64_t)((row / a.S) % a.H) * a.st_sh + (int64_t)((2 * lane) / a.gs) * a.st_sg;
+  const int64_t off = (int64_t)h * a.st_sh + (int64_t)lane_group(a, lane) * a.st_sg;
   return a.st_f32 ? reinterpret_cast<const uint32_t*>(a.st)[off]
                   : (uint32_t)reinterpret_cast<const uint16_t*>(a.st)[off];
 }
@@ -243,23 +299,34 @@ __device__ __forceinline__ float row_static(const AppendDev& a, int row, int lan
   if (a.st == nullptr || a.fmt == KVQ_FMT_INT4_ASYM || a.fmt == KVQ_FMT_INT4_KIVI ||
       a.fmt == KVQ_FMT_INT8_KIVI)
     return 0.f;
-  return ld_static(a, (row / a.S) % a.H, (2 * lane) / a.gs);
+  return ld_static(a, (row / a.S) % a.H, lane_group(a, lane));
 }
 
 // Quantizes append row `row` = (b * H + h) * S + s_idx whose lane values xv (and static
 // scale stv, row_static) were loaded by the caller.  FMT: the side's format when the caller
 // knows it at compile time (the fused decode step's writer: only that format's code is
 // built into its kernel), or -1 for a.fmt.
+// pre: a KIVI K side's frozen parameters of the lane's channels, where the caller requested them
+// ahead (kivi_pre), or NULL.
+struct KiviPre {
+  float s0, s1, z0, z1;
+};
+__device__ __forceinline__ KiviPre kivi_pre(const AppendDev& a, int b, int h, int lane) {
+  const int64_t o = (int64_t)b * a.st_sb + (int64_t)h * a.st_sh + (int64_t)(2 * lane) * a.st_sg;
+  const float* ps = reinterpret_cast<const float*>(a.st);
+  const float* pz = reinterpret_cast<const float*>(a.st_zp);
+  return KiviPre{ps[o], ps[o + a.st_sg], pz[o], pz[o + a.st_sg]};
+}
 template <int FMT = -1>
-__device__ __forceinline__ void quant_row_bhs(const AppendDev& a, int b, int h, int s_idx, int row,
-                                              int lane, float thr, half2v xv, float stv) {
+__device__ __forceinline__ void quant_row_bhs(const AppendDev& a, int b, int h, int s_idx,
+                                              int lane, float thr, half2v xv, float stv,
+                                              const KiviPre* pre = nullptr) {
 #pragma clang fp contract(off)
   const int fmt = FMT >= 0 ? FMT : a.fmt;
   const int64_t t = a.wpos + s_idx;
-  const half_t* xr = row_x(a, row);
   const float x0 = (float)xv.x, x1 = (float)xv.y;
   const int d0 = 2 * lane;
-  const int g = d0 / a.gs;
+  const int g = lane_group(a, lane);
 
   // NaN / Inf detection (src/quant/_common.py:13-20): reported through status[0]
   const bool bad = !(__builtin_isfinite(x0) && __builtin_isfinite(x1));
@@ -269,7 +336,7 @@ __device__ __forceinline__ void quant_row_bhs(const AppendDev& a, int b, int h, 
   // the group's absmax, or for a percentile-clipped dynamic scale its quantile of |x|
   const bool pct = a.st == nullptr && a.dq > 0.f &&
                    (fmt == KVQ_FMT_INT8_SYM || fmt == KVQ_FMT_INT4_SYM);
-  const float am = pct ? group_quantile(fabsf(x0), fabsf(x1), a.gs, a.dq, lane)
+  const float am = pct ? group_quantile(fabsf(x0), fabsf(x1), a.gs, a.dq, lane, !badmask)
                        : group_absmax(fmaxf(fabsf(x0), fabsf(x1)), a.gs);
   uint8_t* crow = a.codes + (int64_t)b * a.csb + (int64_t)h * a.csh + t * a.cst;
   int clipped = 0;
@@ -280,7 +347,7 @@ __device__ __forceinline__ void quant_row_bhs(const AppendDev& a, int b, int h, 
     *reinterpret_cast<uint16_t*>(crow + d0) = int8_pack_pair(x0, x1, s16, clipped);
     // the clip statistic is the static-scale path's (int8_cache.py:401-419)
     if (a.st == nullptr) clipped = 0;
-    if (a.so && (d0 % a.gs) == 0) {
+    if (a.so && (d0 & (a.gs - 1)) == 0) {
       const int64_t off = (int64_t)b * a.sosb + (int64_t)h * a.sosh + t * a.sost + (int64_t)g * a.sosg;
       if (a.so_f32) reinterpret_cast<float*>(a.so)[off] = sf;
       else reinterpret_cast<half_t*>(a.so)[off] = s16;
@@ -301,7 +368,7 @@ __device__ __forceinline__ void quant_row_bhs(const AppendDev& a, int b, int h, 
       const float bound = s * 7.0f;                          // int4_cache.py:473-476
       clipped = (fabsf(x0) > bound) + (fabsf(x1) > bound);
     }
-    if (a.so && (d0 % a.gs) == 0) {
+    if (a.so && (d0 & (a.gs - 1)) == 0) {
       const int64_t off = (int64_t)b * a.sosb + (int64_t)h * a.sosh + t * a.sost + (int64_t)g * a.sosg;
       if (a.so_f32) reinterpret_cast<float*>(a.so)[off] = s;
       else reinterpret_cast<half_t*>(a.so)[off] = (half_t)s;
@@ -313,25 +380,19 @@ __device__ __forceinline__ void quant_row_bhs(const AppendDev& a, int b, int h, 
     float s0, s1, z0, z1;
     if (a.st != nullptr) {
       // K: frozen per-channel parameters (kivi_style_cache.py:548-566)
-      const int64_t o = (int64_t)b * a.st_sb + (int64_t)h * a.st_sh + (int64_t)d0 * a.st_sg;
-      const float* ps = reinterpret_cast<const float*>(a.st);
-      const float* pz = reinterpret_cast<const float*>(a.st_zp);
-      s0 = ps[o]; s1 = ps[o + a.st_sg];
-      z0 = pz[o]; z1 = pz[o + a.st_sg];
+      const KiviPre p = pre ? *pre : kivi_pre(a, b, h, lane);
+      s0 = p.s0; s1 = p.s1;
+      z0 = p.z0; z1 = p.z1;
     } else {
       // V: per-token range over the 128 channels (asymmetric_quant.py:97-141): min / max, or
       // with a percentile below 100 torch.quantile at (100 - p) / 100 and p / 100
       float mn, mx;
       if (a.dq > 0.f) {
-        mn = group_quantile(x0, x1, 128, a.dq_lo, lane);
-        mx = group_quantile(x0, x1, 128, a.dq, lane);
+        mn = group_quantile(x0, x1, 128, a.dq_lo, lane, !badmask);
+        mx = group_quantile(x0, x1, 128, a.dq, lane, !badmask);
       } else {
-        mn = fminf(x0, x1);
-        mx = fmaxf(x0, x1);
-        for (int o = 32; o > 0; o >>= 1) {
-          mn = fminf(mn, __shfl_xor(mn, o, 64));
-          mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-        }
+        mn = -wave_max64(-fminf(x0, x1));
+        mx = wave_max64(fmaxf(x0, x1));
       }
       // range floor max(1e-5, fp16 tiny * (qmax - qmin)) = (qmax - qmin) * 2^-14;
       // z = min - qmin s (qmin s is exact)
@@ -367,7 +428,7 @@ __device__ __forceinline__ void quant_row_bhs(const AppendDev& a, int b, int h, 
     if (a.n_out > 0 && lane < a.n_out) {
       const int ch = min(max(a.oidx[h * a.n_out + lane], 0), 127);
       half_t* orow = a.oo + (int64_t)b * a.oosb + (int64_t)h * a.oosh + t * a.oost;
-      orow[lane] = xr[ch];
+      orow[lane] = row_x_at(a, b, h, s_idx)[ch];
     }
   }
   // clipped-element count (int8_cache.py:407-419, int4_cache.py:468-485)
@@ -381,7 +442,7 @@ __device__ __forceinline__ void quant_row_x(const AppendDev& a, int row, int lan
                                             half2v xv, float stv) {
   const int s_idx = row % a.S;
   const int bh = row / a.S;
-  quant_row_bhs<FMT>(a, bh / a.H, bh % a.H, s_idx, row, lane, thr, xv, stv);
+  quant_row_bhs<FMT>(a, bh / a.H, bh % a.H, s_idx, lane, thr, xv, stv);
 }
 
 
@@ -428,25 +489,85 @@ __host__ __device__ inline bool rescue_walk_ok(float q, int n) {
 // decode step's writer), over at most kRescueRows rows (rows = B * H) in groups of 16 or more.
 // rescue_fetch issues the rows' loads early (lane l: the 32 dwords of channels
 // 64 (l % 2) .. + 63 of row l / 2); rescue_thr_rows then takes each lane's group maxima (a
-// group of 128 with its partner lane), writes the scales fmax(absmax, 1e-5) / 7 to dyn (LDS
-// of this wave alone; a wave barrier orders the writes before the walk's reads) and walks
-// from the top.  Needs
-// rescue_walk_ok(a.rq, rows * 128 / gs).
+// group of 128 with its partner lane).  Where the ranks are the two largest (up to 100 scales at
+// a ratio of 1 %) and every value is finite, neither the LDS nor a division per scale is needed:
+// absmax -> scale is monotone, so the two largest absmax values, found in registers, are all that
+// is scaled.  Elsewhere the scales fmax(absmax, 1e-5) / 7 go to dyn (LDS of this wave alone; a
+// wave barrier orders the writes before the walk's reads) and the walk from the top takes them.
+// Needs rescue_walk_ok(a.rq, rows * 128 / gs).
+// (Fused step of an INT4 cache with a 1 % rescue in groups of 16, 1 x 2 kv heads x 500 tokens:
+// 12.3 -> 10.8 us, of which the attention is 7.3.  16 lanes a row instead, 4 rows a load: 12.8, for
+// the eight row addresses and the group maxima across lanes.)
 constexpr int kRescueRows = 32;
 struct RescueRows {
   uint32_t w[32];
 };
 __device__ __forceinline__ void rescue_fetch(const AppendDev& a, int lane, RescueRows& x) {
-  const int rows = a.B * a.H * a.S, r = lane >> 1;
-  const uint32_t* p = reinterpret_cast<const uint32_t*>(row_x(a, r < rows ? r : 0)) + 32 * (lane & 1);
+  const uint32_t rows = (uint32_t)(a.B * a.H), r = (uint32_t)lane >> 1 < rows ? (uint32_t)lane >> 1 : 0u;
+  const uint32_t H = (uint32_t)a.H, rb = r / H;
+  const uint32_t* p =
+      reinterpret_cast<const uint32_t*>(row_x_at(a, (int)rb, (int)(r - rb * H), 0)) + 32 * (lane & 1);
+  // (every lane reads lines of its own: 8 loads of 16 bytes, where the rows allow, occupy the
+  // address unit a quarter of the time of 32 dwords)
+  if ((uintptr_t)a.x % 16 == 0 && a.xsb % 8 == 0 && a.xsh % 8 == 0) {
 #pragma unroll
-  for (int i = 0; i < 32; ++i) x.w[i] = p[i];
+    for (int i = 0; i < 8; ++i) {
+      const u32x4 v = reinterpret_cast<const u32x4*>(p)[i];
+      x.w[4 * i] = v.x;
+      x.w[4 * i + 1] = v.y;
+      x.w[4 * i + 2] = v.z;
+      x.w[4 * i + 3] = v.w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) x.w[i] = p[i];
+  }
 }
 __device__ __forceinline__ float rescue_thr_rows(const AppendDev& a, int lane, const RescueRows& x,
                                                  float* dyn) {
 #pragma clang fp contract(off)
-  const int rows = a.B * a.H * a.S, gs = a.gs, G = 128 / gs, n = rows * G;
+  const int rows = a.B * a.H, gs = a.gs, G = 128 >> (31 - __builtin_clz(gs)), n = rows * G;
   const int r = lane >> 1, hh = lane & 1;
+  const float rank = a.rq * (float)(n - 1);
+  const int lo = (int)floorf(rank), hi = (int)ceilf(rank);
+  const float w = rank - (float)lo;
+  if (lo >= n - 2) {
+    uint32_t k16[4];  // |x| of the lane's four runs of 16 channels, as fp16 bits (ordered as integers)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      uint32_t m = x.w[8 * k] & 0x7FFF7FFFu;
+#pragma unroll
+      for (int i = 1; i < 8; ++i) m = pk_max_u(m, x.w[8 * k + i] & 0x7FFF7FFFu);
+      k16[k] = max(m & 0xFFFFu, m >> 16);
+    }
+    if (!__any(max(max(k16[0], k16[1]), max(k16[2], k16[3])) >= 0x7C00u)) {
+      float f[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) f[k] = (float)__builtin_bit_cast(half_t, (uint16_t)k16[k]);
+      float t1, t2 = -1.0f;  // the lane's two largest groups (-1: below every absmax)
+      if (gs >= 64) {
+        t1 = fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3]));
+        if (gs == 128) {  // with the partner lane's half
+          t1 = fmaxf(t1, dppf<0xB1>(t1));
+          if (hh != 0) t1 = -1.0f;
+        }
+      } else if (gs == 32) {
+        const float g0 = fmaxf(f[0], f[1]), g1 = fmaxf(f[2], f[3]);
+        t1 = fmaxf(g0, g1);
+        t2 = fminf(g0, g1);
+      } else {
+        const float h0 = fmaxf(f[0], f[1]), l0 = fminf(f[0], f[1]);
+        const float h1 = fmaxf(f[2], f[3]), l1 = fminf(f[2], f[3]);
+        t1 = fmaxf(h0, h1);
+        t2 = fmaxf(fminf(h0, h1), fmaxf(l0, l1));
+      }
+      if (r >= rows) t1 = t2 = -1.0f;
+      group_top2(t1, t2, 128, lane, t1, t2);
+      t1 = __fdiv_rn(fmaxf(t1, 1e-5f), 7.0f);
+      t2 = __fdiv_rn(fmaxf(t2, 1e-5f), 7.0f);
+      return quantile_lerp(lo == n - 1 ? t1 : t2, hi == n - 1 ? t1 : t2, w);
+    }
+  }
   float m16[4];  // the maxima of |x| over the lane's four runs of 16 channels
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -482,9 +603,6 @@ __device__ __forceinline__ float rescue_thr_rows(const AppendDev& a, int lane, c
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const float rank = a.rq * (float)(n - 1);
-  const int lo = (int)floorf(rank), hi = (int)ceilf(rank);
-  const float w = rank - (float)lo;
   return n <= 64    ? wave_top_quantile<1>(dyn, n, lo, hi, w, lane)
          : n <= 128 ? wave_top_quantile<2>(dyn, n, lo, hi, w, lane)
                     : wave_top_quantile<4>(dyn, n, lo, hi, w, lane);

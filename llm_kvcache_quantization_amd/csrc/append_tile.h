@@ -9,13 +9,8 @@ namespace kvq {
 
 namespace {
 
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ uint32_t pk_max_u(uint32_t a, uint32_t b) {
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a),
-                                                                __builtin_bit_cast(u16x2, b)));
-}
 __device__ __forceinline__ uint32_t pk_max_i(uint32_t a, uint32_t b) {
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(i16x2, a),
                                                                 __builtin_bit_cast(i16x2, b)));

@@ -2117,14 +2117,21 @@ __device__ __forceinline__ bool rescue_side(const AppendDev& d) {
 struct RowPre {
   half2v k, v;
   uint32_t sk, sv;  // the static scales' bits (row_static_bits)
+  KiviPre kk;       // KIVI K: the frozen parameters
 };
+// KIVI K with frozen parameters (else its parameters are the token's own)
+template <int KFMT>
+__device__ __forceinline__ bool kivi_frozen(const AppendDev& a) {
+  return (KFMT == KVQ_FMT_INT4_KIVI || KFMT == KVQ_FMT_INT8_KIVI) && a.st != nullptr;
+}
+template <int KFMT>
 __device__ __forceinline__ void append_row_fetch(const DecodeArgs& a, int b, int hkv, int lane,
                                                  RowPre& p) {
-  const int row = b * a.ark.H + hkv;
-  p.k = load_x(a.ark, row, lane);
-  p.sk = row_static_bits(a.ark, row, lane);
-  p.v = load_x(a.arv, row, lane);
-  p.sv = row_static_bits(a.arv, row, lane);
+  p.k = *reinterpret_cast<const half2v*>(row_x_at(a.ark, b, hkv, 0) + 2 * lane);
+  p.sk = row_static_bits(a.ark, hkv, lane);
+  if (kivi_frozen<KFMT>(a.ark)) p.kk = kivi_pre(a.ark, b, hkv, lane);
+  p.v = *reinterpret_cast<const half2v*>(row_x_at(a.arv, b, hkv, 0) + 2 * lane);
+  p.sv = row_static_bits(a.arv, hkv, lane);
 }
 // (the rescue is compiled only where it can occur: INT4_SYM K and V, RESCUE)
 // KFMT / VFMT: the sides' formats (the kernel's operand types; the host admits only appends
@@ -2134,19 +2141,19 @@ template <bool RESCUE, int KFMT, int VFMT>
 __device__ __forceinline__ void append_row_pair(const DecodeArgs& a, int b, int hkv, int lane,
                                                 const RowPre& p, const RescueRows& rk,
                                                 const RescueRows& rv) {
-  const int row = b * a.ark.H + hkv;
+  const KiviPre* const kk = kivi_frozen<KFMT>(a.ark) ? &p.kk : nullptr;
   float tk = 0.f, tv = 0.f;
   if constexpr (RESCUE) {
     // the writer's scales of each side (one writer per work-group; one array per side, so the
     // V side's writes cannot pass the K side's reads)
     __shared__ float rdyn_k[kRescueRows * 8], rdyn_v[kRescueRows * 8];
     if (rescue_side(a.ark)) tk = rescue_thr_rows(a.ark, lane, rk, rdyn_k);
-    quant_row_bhs<KFMT>(a.ark, b, hkv, 0, row, lane, tk, p.k, static_value(a.ark, p.sk));
+    quant_row_bhs<KFMT>(a.ark, b, hkv, 0, lane, tk, p.k, static_value(a.ark, p.sk), kk);
     if (rescue_side(a.arv)) tv = rescue_thr_rows(a.arv, lane, rv, rdyn_v);
   } else {
-    quant_row_bhs<KFMT>(a.ark, b, hkv, 0, row, lane, tk, p.k, static_value(a.ark, p.sk));
+    quant_row_bhs<KFMT>(a.ark, b, hkv, 0, lane, tk, p.k, static_value(a.ark, p.sk), kk);
   }
-  quant_row_bhs<VFMT>(a.arv, b, hkv, 0, row, lane, tv, p.v, static_value(a.arv, p.sv));
+  quant_row_bhs<VFMT>(a.arv, b, hkv, 0, lane, tv, p.v, static_value(a.arv, p.sv));
 }
 
 __device__ __forceinline__ void append_status(const FusedAppend& f, const AppendFlags& fl) {
@@ -2457,7 +2464,7 @@ void decode_tiled_kernel(DecodeArgs a) {
   kf.fetch_q(a, bq, hkv, lane, wave, qin);
   if constexpr (KF::kAppendRow) {
     if (writer) {
-      append_row_fetch(a, b, hkv, lane, rpre);
+      append_row_fetch<KF::kRowFmt>(a, b, hkv, lane, rpre);
       if constexpr (KF::kRescue)
         if (rescue_side(a.ark) || rescue_side(a.arv)) {
           rescue_fetch(a.ark, lane, rxk);
