@@ -184,8 +184,10 @@ def lib() -> ctypes.CDLL:
         L.kvq_abi_version.restype = c_i32
         # the engines' own entry points (csrc/engine_ops.h), no part of the public ABI
         L.kvq_kivi_channel_range.argtypes = [c_vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_i32, c_i32,
-                                             c_f32, c_f32, c_vp, c_vp, c_vp]
+                                             c_f32, c_f32, c_vp, c_vp, c_vp, c_i64, c_vp]
         L.kvq_kivi_channel_range.restype = c_i32
+        L.kvq_kivi_range_scratch_bytes.argtypes = [c_i32, c_i32, c_i32, c_f32]
+        L.kvq_kivi_range_scratch_bytes.restype = c_i64
         pv = ctypes.POINTER(KvView)
         L.kvq_dequant.argtypes = [pv, c_i32, c_i32, c_vp, pv, c_i32, c_i32, c_vp, c_i32, c_i32, c_i32, c_vp]
         L.kvq_dequant.restype = c_i32

@@ -1278,7 +1278,7 @@ def kivi_channel_params(k: Tensor, bits: int, percentile: float) -> Tuple[Tensor
     """Per-channel K scale / zero-point over the tokens of a prefill k [B, H, S, D]
     (quantize_asymmetric_per_channel, src/quant/asymmetric_quant.py:24-141, 199-224): the
     range (min / max, or the two quantiles) in fp32, floored at max(1e-5, fp16 tiny x
-    (qmax - qmin)), divided by qmax - qmin; z = min - qmin s.  fp32 [B, H, D].  One HIP launch
+    (qmax - qmin)), divided by qmax - qmin; z = min - qmin s.  fp32 [B, H, D].  One or two HIP launches
     for fp16 rows on the GPU (kvq_kivi_channel_range)."""
     qmin, qmax = (-8, 7) if bits == 4 else (-128, 127)
     lo_q, hi_q = _kivi_levels(percentile)
@@ -1287,9 +1287,12 @@ def kivi_channel_params(k: Tensor, bits: int, percentile: float) -> Tuple[Tensor
         B, H, S, D = k.shape
         s = torch.empty(B, H, D, dtype=torch.float32, device=k.device)
         z = torch.empty_like(s)
-        C.check(C.lib().kvq_kivi_channel_range(k.data_ptr(), *k.stride()[:3], B, H, S, bits, lo_q, hi_q,
-                                               s.data_ptr(), z.data_ptr(),
-                                               ctypes.c_void_p(C.stream_handle(k.device))))
+        lib = C.lib()
+        n = lib.kvq_kivi_range_scratch_bytes(B, H, S, hi_q)
+        part = torch.empty(n, dtype=torch.uint8, device=k.device) if n else None
+        C.check(lib.kvq_kivi_channel_range(k.data_ptr(), *k.stride()[:3], B, H, S, bits, lo_q, hi_q,
+                                           s.data_ptr(), z.data_ptr(), part.data_ptr() if n else None, n,
+                                           ctypes.c_void_p(C.stream_handle(k.device))))
         return s, z
     kf = k.float()
     if hi_q > 0.0:
@@ -1314,7 +1317,7 @@ class _KiviFamily(_EngineBase):
     parameters); a 16-bit side keeps fp16 values.  Codes: 4 bits packed [B, H, T, 64] (byte =
     ((c[2i]+8) << 4) | (c[2i+1]+8)), 8 bits int8 [B, H, T, 128].  Every quantized token goes
     through kvq_quant_append (HIP; per-token percentile clipping in the kernel); the prefill's
-    per-channel K range is one HIP launch (:func:`kivi_channel_params`).  Decode attention reads the cache in place through the
+    per-channel K range is a HIP launch or two (:func:`kivi_channel_params`).  Decode attention reads the cache in place through the
     tiled kernel of the layer's pair (kvq_decode_attn), the fp16 residual window (residual_length
     > 0) with it, merged by the kernel's merging work-group.
     """

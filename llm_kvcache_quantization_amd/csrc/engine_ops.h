@@ -14,10 +14,13 @@ extern "C" {
 // tokens of x fp16 [B, H, S, 128] (strides in elements, channels contiguous, 4-byte aligned
 // rows), the minimum and maximum (q_hi = 0) or torch.quantile at the levels q_lo, q_hi, then
 // s = max(range, max(1e-5, 2^-14 span)) / span with span = 15 (bits 4) or 255 (bits 8), and
-// z = min + (span + 1) / 2 s; fp32 [B, H, 128] dense.
+// z = min + (span + 1) / 2 s; fp32 [B, H, 128] dense.  scratch: device memory of
+// kvq_kivi_range_scratch_bytes (0: none is used), 4-byte aligned, any contents; without it the
+// same result comes from one launch.
+int64_t kvq_kivi_range_scratch_bytes(int32_t batch, int32_t heads, int32_t tokens, float q_hi);
 int kvq_kivi_channel_range(const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_s, int32_t batch,
                            int32_t heads, int32_t tokens, int32_t bits, float q_lo, float q_hi, float* scale,
-                           float* zero_point, kvq_stream_t stream);
+                           float* zero_point, void* scratch, int64_t scratch_bytes, kvq_stream_t stream);
 
 // Dequantised fp16 rows [B, H, tokens, 128] (dense) of K and V views (either NULL: left out) in
 // the formats INT8_SYM / INT4_SYM (scale views as kvq_decode_attn takes them, any strides, in

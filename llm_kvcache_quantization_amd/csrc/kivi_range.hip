@@ -1,7 +1,7 @@
 // Per-channel ranges of a prompt's K (the frozen parameters of the KIVI layout).
 //
-// One work-group takes 8 channels of one (b, head) over all tokens, so nothing is merged between
-// work-groups and the whole reduction is one launch: a thread reads 16 bytes of a token's row.
+// Percentiles, and min / max up to range_splits: one work-group takes 8 channels of one (b, head)
+// over all tokens, so nothing is merged between work-groups and the whole reduction is one launch: a thread reads 16 bytes of a token's row.
 // The 16 work-groups of a (b, head) run on one XCD (work-group ids go round the 8 XCDs), whose L2
 // then fetches each row once for all of them.
 //
@@ -12,10 +12,10 @@
 // again (L2, or the Infinity Cache).
 //
 // Bound: few units leave CUs idle, and a CU takes about two cycles for the 128-byte line of every
-// row (1 x 2 heads x 32768 tokens: 40 us for min / max); then the LDS atomics of the first
-// histogram.  4 heads x 8191 tokens: min / max 8.8 us (torch's aminmax of the fp32 copy 48 us at
-// 1999 tokens), 99.9 percentiles 20.7 us (torch.sort in fp32 with index arrays, transposes and
-// casts about 300 us); 8 x 4 heads x 32768: 85 and 178 us.
+// row (1 x 2 heads x 32768 tokens: 40 us for min / max, why long prompts split it); then the LDS
+// atomics of the first histogram.  4 heads x 1999 tokens: min / max 4.8 us (torch's aminmax of the
+// fp32 copy 48 us); 4 x 8191: 99.9 percentiles 20.7 us (torch.sort in fp32 with index arrays,
+// transposes and casts about 300 us); 8 x 4 heads x 32768: 178 us, min / max 48 us (5.6 TB/s).
 #include "append_tile.h"
 #include "engine_ops.h"
 
@@ -28,6 +28,7 @@ namespace {
 constexpr int kRows = 8;    // rows a thread holds
 constexpr int kCopies = 4;  // copies of the upper-byte histogram: the values crowd in a few bins
 constexpr int kStride = 257;
+constexpr int kSplitGroups = 2048;  // work-groups of the split min / max: 8 of 256 threads a CU
 
 struct RangeArgs {
   const half_t* x;
@@ -37,6 +38,8 @@ struct RangeArgs {
   int r[4];         // ranks: lower tail floor / ceil, upper tail floor / ceil
   float wl, wh;
   float *scale, *zp;
+  uint32_t* part;   // min / max by splits: [units, splits, 2, 64] packed keys
+  int splits;
 };
 
 // fp16 bits -> 16-bit unsigned keys in the order of the values, every NaN above them all
@@ -187,6 +190,83 @@ __global__ __launch_bounds__(1024) void kivi_range_kernel(RangeArgs a) {
   }
 }
 
+// Min / max of a long prompt in two launches: work-groups of whole rows over all CUs (a wave reads
+// four rows an instruction), each leaving the largest keys and largest ~keys of its tokens, then
+// one work-group a unit over those.  Bound: the rows' bytes, plus the second launch (about 4 us).
+template <RowLoad LD>
+__global__ __launch_bounds__(256) void kivi_range_part_kernel(RangeArgs a) {
+  const int split = (int)blockIdx.x % a.splits, unit = (int)blockIdx.x / a.splits;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = threadIdx.x & 15;
+  const int chunk = ((a.S + a.splits - 1) / a.splits + 127) / 128 * 128;  // tokens of a work-group
+  const int end = min(a.S, (split + 1) * chunk);
+  const half_t* xr = a.x + (int64_t)(unit / a.H) * a.sb + (int64_t)(unit % a.H) * a.sh + 8 * c;
+  __shared__ uint32_t red[4][2][64];
+  uint32_t hi[4] = {0, 0, 0, 0}, lo[4] = {0, 0, 0, 0};  // (an empty split leaves these)
+  for (int s0 = split * chunk; s0 < end; s0 += 128) {
+    u32x4 w[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)  // rows past the end repeat the last one
+      w[i] = ld_row<LD>(xr + (int64_t)min(s0 + 16 * i + (int)(threadIdx.x >> 4), end - 1) * a.ss);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t k = key2(w[i][j]);
+        hi[j] = pk_max_u(hi[j], k);
+        lo[j] = pk_max_u(lo[j], ~k);
+      }
+  }
+#pragma unroll
+  for (int o = 16; o < 64; o <<= 1)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      hi[j] = pk_max_u(hi[j], (uint32_t)__shfl_xor((int)hi[j], o, 64));
+      lo[j] = pk_max_u(lo[j], (uint32_t)__shfl_xor((int)lo[j], o, 64));
+    }
+  if (lane < 16)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) red[wave][0][4 * c + j] = hi[j], red[wave][1][4 * c + j] = lo[j];
+  __syncthreads();
+  if (threadIdx.x < 128) {
+    const uint32_t* r = &red[0][0][threadIdx.x];
+    a.part[(int64_t)blockIdx.x * 128 + threadIdx.x] =
+        pk_max_u(pk_max_u(r[0], r[128]), pk_max_u(r[256], r[384]));
+  }
+}
+
+__global__ __launch_bounds__(1024) void kivi_range_merge_kernel(RangeArgs a) {
+  const int unit = blockIdx.x, col = threadIdx.x & 127, grp = threadIdx.x >> 7;
+  const uint32_t* p = a.part + (int64_t)unit * a.splits * 128 + col;
+  __shared__ uint32_t red[8][128];
+  uint32_t m = 0;
+  for (int i = grp; i < a.splits; i += 8) m = pk_max_u(m, p[(int64_t)i * 128]);
+  red[grp][col] = m;
+  __syncthreads();
+  if (threadIdx.x < 128) {
+    const int pair = threadIdx.x >> 1, sft = 16 * (threadIdx.x & 1);
+    uint32_t h = 0, l = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      h = max(h, (red[i][pair] >> sft) & 0xFFFFu);
+      l = max(l, (red[i][64 + pair] >> sft) & 0xFFFFu);
+    }
+    const float mx = value_of(h);
+    store_range(a, (int64_t)unit * 128 + threadIdx.x, h == 0xFFFFu ? mx : value_of(~l & 0xFFFFu), mx);
+  }
+}
+
+// Work-groups a unit of the split min / max, or 0 for the single launch.  One launch against two, us:
+// 1 x 2 heads x 1024 tokens 4.5 / 6.4, 1 x 4 x 1999 4.8 / 6.4, 1 x 2 x 4096 7.7 / 6.6 (a second
+// launch also costs the host about 4), 1 x 4 x 8191 9.8 / 7.2, 8 x 8 x 1024 9.0 / 7.3, 4 x 8 x 4096
+// 15.6 / 9.4, 1 x 2 x 32768 39.7 / 10.8, 8 x 8 x 8192 46.7 / 26.7, 8 x 4 x 32768 84.2 / 47.8: it pays
+// where a unit's 16 CUs read long, or where the units' rows are many.
+int range_splits(int64_t units, int tokens) {
+  if (units <= 0 || tokens > (1 << 30)) return 0;
+  if (tokens <= 8192 && (tokens < 1024 || units * tokens < 65536)) return 0;
+  const int64_t most = ((int64_t)tokens + 255) / 256, fill = (kSplitGroups + units - 1) / units;
+  return (int)(fill < most ? fill : most);
+}
+
 template <bool PCT>
 void launch_range(const RangeArgs& a, bool al16, hipStream_t st) {
   const dim3 grid((unsigned)((a.units + 7) / 8 * 128));
@@ -203,9 +283,16 @@ void launch_range(const RangeArgs& a, bool al16, hipStream_t st) {
 
 using namespace kvq;
 
+extern "C" int64_t kvq_kivi_range_scratch_bytes(int32_t batch, int32_t heads, int32_t tokens, float q_hi) {
+  const int64_t units = batch > 0 && heads > 0 ? (int64_t)batch * heads : 0;
+  const int n = q_hi == 0.f && units <= (1 << 20) ? range_splits(units, tokens) : 0;
+  return n > 1 ? units * n * 128 * (int64_t)sizeof(uint32_t) : 0;
+}
+
 extern "C" int kvq_kivi_channel_range(const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_s,
                                       int32_t batch, int32_t heads, int32_t tokens, int32_t bits, float q_lo,
-                                      float q_hi, float* scale, float* zero_point, kvq_stream_t stream) {
+                                      float q_hi, float* scale, float* zero_point, void* scratch,
+                                      int64_t scratch_bytes, kvq_stream_t stream) {
   if (!x || !scale || !zero_point) return fail(KVQ_ERR_INVALID, "channel range: NULL pointer");
   if (batch < 0 || heads < 0 || tokens <= 0 || (int64_t)batch * heads > (1 << 20))
     return fail(KVQ_ERR_INVALID, "channel range: bad shape");
@@ -226,7 +313,17 @@ extern "C" int kvq_kivi_channel_range(const void* x, int64_t stride_b, int64_t s
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool al16 = (uintptr_t)x % 16 == 0 && stride_b % 8 == 0 && stride_h % 8 == 0 && stride_s % 8 == 0;
   if (q_hi == 0.f) {
-    launch_range<false>(a, al16, st);
+    a.splits = range_splits(a.units, a.S);
+    a.part = reinterpret_cast<uint32_t*>(scratch);
+    if (a.splits > 1 && scratch && (uintptr_t)scratch % 4 == 0 &&
+        scratch_bytes >= kvq_kivi_range_scratch_bytes(batch, heads, tokens, q_hi)) {
+      const dim3 grid((unsigned)(a.units * a.splits));
+      if (al16) hipLaunchKernelGGL((kivi_range_part_kernel<kCached>), grid, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL((kivi_range_part_kernel<kDwords>), grid, dim3(256), 0, st, a);
+      hipLaunchKernelGGL(kivi_range_merge_kernel, dim3((unsigned)a.units), dim3(1024), 0, st, a);
+    } else {
+      launch_range<false>(a, al16, st);
+    }
   } else {
     // torch.quantile's fp32 ranks; ceil of a rank that rounded up to n - 1 stays in range
     const float n1 = (float)(tokens - 1), rl = q_lo * n1, rh = q_hi * n1;

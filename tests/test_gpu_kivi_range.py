@@ -80,3 +80,33 @@ def test_prefill_rejects_nan_and_keeps_no_parameters():
     cache.clear()
     cache.append(0, k, k)
     assert cache.get_seq_len() == 40
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 8193), (2, 32, 1024), (3, 5, 4370), (1, 2, 33000), (16, 9, 1100)], ids=str)
+def test_split_range_equals_one_launch(shape):
+    """Long prompts in two launches over splits of the tokens: the same bits as the single launch
+    (no scratch), for dense, transposed and 4-byte aligned rows, with NaN and Inf."""
+    import ctypes
+
+    from llm_kvcache_quantization_amd import _capi as C
+
+    L = C.lib()
+    B, H, S = shape
+    n = L.kvq_kivi_range_scratch_bytes(B, H, S, 0.0)
+    assert n > 0 and L.kvq_kivi_range_scratch_bytes(B, H, S, 0.999) == 0
+    k = _k(B, H, S, 3).cuda()
+    k[0, 0, S - 1, 3], k[-1, -1, 0, 9], k[-1, 0, S // 2, 70] = float("nan"), float("inf"), -float("inf")
+    t = k.transpose(1, 2).contiguous().transpose(1, 2)
+    odd = torch.zeros(B, H, S, 130, dtype=torch.float16, device="cuda")[..., 2:]
+    odd.copy_(k)
+    for x in (k, t, odd):
+        res = []
+        for m in (n, 0):
+            part = torch.full((n + 256,), 0xA5, dtype=torch.uint8, device="cuda")
+            s, z = (torch.full((B, H, 128), -7.0, device="cuda") for _ in range(2))
+            C.check(L.kvq_kivi_channel_range(x.data_ptr(), *x.stride()[:3], B, H, S, 8, 0.0, 0.0, s.data_ptr(),
+                                             z.data_ptr(), part.data_ptr() if m else None, m,
+                                             ctypes.c_void_p(C.stream_handle(x.device))))
+            assert bool((part[n:] == 0xA5).all())
+            res.append(torch.stack([s, z]).view(torch.int32))
+        assert torch.equal(res[0], res[1])
