@@ -485,19 +485,51 @@ __host__ __device__ inline bool rescue_walk_ok(float q, int n) {
   return n - 1 - lo < kTopWalk;
 }
 
+// The four largest values of the wave (t: each lane's own, descending; afterwards every lane holds
+// the wave's).  Two descending fours merge by the larger of each value and the other four's
+// reverse, which is bitonic, then two rounds of exchanges.
+__device__ __forceinline__ void merge_top4(float t[4], float n0, float n1, float n2, float n3) {
+  const float a = fmaxf(t[0], n3), b = fmaxf(t[1], n2), c = fmaxf(t[2], n1), d = fmaxf(t[3], n0);
+  const float a1 = fmaxf(a, c), c1 = fminf(a, c), b1 = fmaxf(b, d), d1 = fminf(b, d);
+  t[0] = fmaxf(a1, b1);
+  t[1] = fminf(a1, b1);
+  t[2] = fmaxf(c1, d1);
+  t[3] = fminf(c1, d1);
+}
+template <int CTRL>
+__device__ __forceinline__ void merge_top4_dpp(float t[4]) {
+  merge_top4(t, dppf<CTRL>(t[0]), dppf<CTRL>(t[1]), dppf<CTRL>(t[2]), dppf<CTRL>(t[3]));
+}
+__device__ __forceinline__ void wave_top4(float t[4]) {
+  merge_top4_dpp<0xB1>(t);   // quad_perm [1, 0, 3, 2]
+  merge_top4_dpp<0x4E>(t);   // quad_perm [2, 3, 0, 1]
+  merge_top4_dpp<0x141>(t);  // row_half_mirror
+  merge_top4_dpp<0x140>(t);  // row_mirror
+  float u[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) u[i] = row_lane(t[i], 0);
+#pragma unroll
+  for (int r = 16; r < 64; r += 16)
+    merge_top4(u, row_lane(t[0], r), row_lane(t[1], r), row_lane(t[2], r), row_lane(t[3], r));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) t[i] = u[i];
+}
+
 // The group-rescue threshold of a one-token append side found by one wave alone (the fused
 // decode step's writer), over at most kRescueRows rows (rows = B * H) in groups of 16 or more.
 // rescue_fetch issues the rows' loads early (lane l: the 32 dwords of channels
 // 64 (l % 2) .. + 63 of row l / 2); rescue_thr_rows then takes each lane's group maxima (a
-// group of 128 with its partner lane).  Where the ranks are the two largest (up to 100 scales at
-// a ratio of 1 %) and every value is finite, neither the LDS nor a division per scale is needed:
-// absmax -> scale is monotone, so the two largest absmax values, found in registers, are all that
-// is scaled.  Elsewhere the scales fmax(absmax, 1e-5) / 7 go to dyn (LDS of this wave alone; a
-// wave barrier orders the writes before the walk's reads) and the walk from the top takes them.
-// Needs rescue_walk_ok(a.rq, rows * 128 / gs).
-// (Fused step of an INT4 cache with a 1 % rescue in groups of 16, 1 x 2 kv heads x 500 tokens:
-// 12.3 -> 10.8 us, of which the attention is 7.3.  16 lanes a row instead, 4 rows a load: 12.8, for
-// the eight row addresses and the group maxima across lanes.)
+// group of 128 with its partner lane).  Where the ranks are among the four largest (every batch up
+// to 32 rows at a ratio of 1 %) and every value is finite, neither the LDS nor a division per
+// scale is needed: absmax -> scale is monotone, so the largest absmax values, found in registers,
+// are all that is scaled.  Elsewhere the scales fmax(absmax, 1e-5) / 7 go to dyn (LDS of this wave
+// alone; a wave barrier orders the writes before the walk's reads) and the walk from the top takes
+// them.  Needs rescue_walk_ok(a.rq, rows * 128 / gs).
+// (Fused step of an INT4 cache with a 1 % rescue in groups of 16, us, with the LDS walk / now /
+// attention alone: 1 x 2 kv heads x 500 tokens 12.3 / 11.0 / 7.3; 8 x 4 x 2000, ranks 252 and 253 of
+// 256, 14.3 / 12.6 / 8.3; 4 x 8 x 8000 16.5 / 15.2 / 13.9.  Only the two largest: 10.8 at the first
+// and the walk at the others; a branch between both won nothing there.  16 lanes a row, 4 rows a
+// load: 12.8 at the first, for the eight row addresses and the group maxima across lanes.)
 constexpr int kRescueRows = 32;
 struct RescueRows {
   uint32_t w[32];
@@ -531,7 +563,7 @@ __device__ __forceinline__ float rescue_thr_rows(const AppendDev& a, int lane, c
   const float rank = a.rq * (float)(n - 1);
   const int lo = (int)floorf(rank), hi = (int)ceilf(rank);
   const float w = rank - (float)lo;
-  if (lo >= n - 2) {
+  if (lo >= n - 4) {
     uint32_t k16[4];  // |x| of the lane's four runs of 16 channels, as fp16 bits (ordered as integers)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -544,28 +576,30 @@ __device__ __forceinline__ float rescue_thr_rows(const AppendDev& a, int lane, c
       float f[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) f[k] = (float)__builtin_bit_cast(half_t, (uint16_t)k16[k]);
-      float t1, t2 = -1.0f;  // the lane's two largest groups (-1: below every absmax)
+      float t[4] = {f[0], -1.0f, -1.0f, -1.0f};  // the lane's groups, descending (-1: none)
       if (gs >= 64) {
-        t1 = fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3]));
+        t[0] = fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3]));
         if (gs == 128) {  // with the partner lane's half
-          t1 = fmaxf(t1, dppf<0xB1>(t1));
-          if (hh != 0) t1 = -1.0f;
+          t[0] = fmaxf(t[0], dppf<0xB1>(t[0]));
+          if (hh != 0) t[0] = -1.0f;
         }
       } else if (gs == 32) {
         const float g0 = fmaxf(f[0], f[1]), g1 = fmaxf(f[2], f[3]);
-        t1 = fmaxf(g0, g1);
-        t2 = fminf(g0, g1);
+        t[0] = fmaxf(g0, g1);
+        t[1] = fminf(g0, g1);
       } else {
         const float h0 = fmaxf(f[0], f[1]), l0 = fminf(f[0], f[1]);
         const float h1 = fmaxf(f[2], f[3]), l1 = fminf(f[2], f[3]);
-        t1 = fmaxf(h0, h1);
-        t2 = fmaxf(fminf(h0, h1), fmaxf(l0, l1));
+        const float x1 = fminf(h0, h1), x2 = fmaxf(l0, l1);
+        t[0] = fmaxf(h0, h1);
+        t[1] = fmaxf(x1, x2);
+        t[2] = fminf(x1, x2);
+        t[3] = fminf(l0, l1);
       }
-      if (r >= rows) t1 = t2 = -1.0f;
-      group_top2(t1, t2, 128, lane, t1, t2);
-      t1 = __fdiv_rn(fmaxf(t1, 1e-5f), 7.0f);
-      t2 = __fdiv_rn(fmaxf(t2, 1e-5f), 7.0f);
-      return quantile_lerp(lo == n - 1 ? t1 : t2, hi == n - 1 ? t1 : t2, w);
+      if (r >= rows) t[0] = t[1] = t[2] = t[3] = -1.0f;
+      wave_top4(t);
+      auto at = [&](int rk) { return rk >= n - 1 ? t[0] : rk == n - 2 ? t[1] : rk == n - 3 ? t[2] : t[3]; };
+      return quantile_lerp(__fdiv_rn(fmaxf(at(lo), 1e-5f), 7.0f), __fdiv_rn(fmaxf(at(hi), 1e-5f), 7.0f), w);
     }
   }
   float m16[4];  // the maxima of |x| over the lane's four runs of 16 channels

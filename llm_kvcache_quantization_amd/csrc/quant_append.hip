@@ -385,7 +385,7 @@ extern "C" int kvq_quant_append(const kvq_append_params* k, const kvq_append_par
   if (!dk.valid && !dv.valid) return KVQ_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // the group rescue takes its threshold from one work-group's LDS sort when every side
-  // that needs one has at most kRescueMax scales, else from the radix select (scratch)
+  // that needs one has at most kRescueMax scales, else from the key select (scratch)
   const bool large = (needs_rescue(k) && rescue_n(k) > kRescueMax) ||
                      (needs_rescue(v) && rescue_n(v) > kRescueMax);
   if (large) {
