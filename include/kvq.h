@@ -119,7 +119,8 @@ typedef struct kvq_kv_view {
  *  - INT8_SYM K whose scale view is static (stride 0, or size 1, over b and t; 128-byte dense
  *    rows) with TILE32 INT4_ASYM V (group 32) or a static INT8_SYM V in dense rows (any
  *    group size);
- *  - per-token INT8_SYM / INT4_SYM scales on both sides in dense rows (groups of 16 or more),
+ *  - per-token INT8_SYM (fp16) / INT4_SYM (fp32 or fp16) scales on both sides in dense rows
+ *    (groups of 16 or more),
  *    INT8_SYM K with per-token scales and INT4_KIVI or FP16 V;
  *  - the KIVI family (INT4_KIVI, INT8_KIVI, FP16 on either side), per-token INT4_KIVI K with
  *    INT4_KIVI, INT8_SYM or FP16 V, and FP16 K with INT8_SYM V.
@@ -258,7 +259,7 @@ typedef struct kvq_append_params {
 /* Appends K and V of one layer with one launch (either pointer may be NULL).  The INT4_SYM
  * group rescue takes torch.quantile's threshold over the dynamic group scales of the whole
  * call (src/cache/int4_cache.py:384-390): up to 4096 (row, group) scales inside the launch,
- * beyond that by an exact radix select over p->scratch (a few short launches first). */
+ * beyond that by an exact select over p->scratch (four short launches first). */
 int kvq_quant_append(const kvq_append_params* k, const kvq_append_params* v,
                      kvq_stream_t stream);
 /* bytes of scratch kvq_quant_append needs for p (0: none) */
@@ -282,8 +283,8 @@ int64_t kvq_append_scratch_bytes(const kvq_append_params* p);
  *    rows: a static scale table and no scale policy (adaptive, rescue, scale_out); an
  *    INT4_ASYM side must name p's static tables and outlier side-band, an INT8_SYM side
  *    quantizes with its own table (fp16 or fp32), as kvq_quant_append would;
- *  - the row formats (per-token INT8_SYM / INT4_SYM scales in dense rows with groups of 16
- *    or more, INT4_KIVI / INT8_KIVI, FP16 sides): any policy kvq_quant_append takes; the
+ *  - the row formats (per-token INT8_SYM fp16 / INT4_SYM fp32 scales in dense rows with groups
+ *    of 16 or more, INT4_KIVI / INT8_KIVI, FP16 sides): any policy kvq_quant_append takes; the
  *    INT4_SYM group rescue with a threshold (rescue_quantile > 0 without rescue_all), which
  *    spans every row of the append, only with at most 32 rows (batch * heads) and its lower
  *    rank within 32 of the top of the (row, group) scales; scale_out / zp_out and KIVI K's
