@@ -302,12 +302,7 @@ __device__ __forceinline__ float row_static(const AppendDev& a, int row, int lan
   return ld_static(a, (row / a.S) % a.H, lane_group(a, lane));
 }
 
-// Quantizes append row `row` = (b * H + h) * S + s_idx whose lane values xv (and static
-// scale stv, row_static) were loaded by the caller.  FMT: the side's format when the caller
-// knows it at compile time (the fused decode step's writer: only that format's code is
-// built into its kernel), or -1 for a.fmt.
-// pre: a KIVI K side's frozen parameters of the lane's channels, where the caller requested them
-// ahead (kivi_pre), or NULL.
+// A KIVI K side's frozen parameters of the lane's two channels
 struct KiviPre {
   float s0, s1, z0, z1;
 };
@@ -317,6 +312,12 @@ __device__ __forceinline__ KiviPre kivi_pre(const AppendDev& a, int b, int h, in
   const float* pz = reinterpret_cast<const float*>(a.st_zp);
   return KiviPre{ps[o], ps[o + a.st_sg], pz[o], pz[o + a.st_sg]};
 }
+
+// Quantizes the append's token s_idx of (b, h), whose lane values xv (and static scale stv,
+// row_static) were loaded by the caller.  FMT: the side's format when the caller
+// knows it at compile time (the fused decode step's writer: only that format's code is
+// built into its kernel), or -1 for a.fmt.  pre: a KIVI K side's frozen parameters where the
+// caller requested them ahead (kivi_pre), or NULL.
 template <int FMT = -1>
 __device__ __forceinline__ void quant_row_bhs(const AppendDev& a, int b, int h, int s_idx,
                                               int lane, float thr, half2v xv, float stv,
