@@ -299,8 +299,9 @@ extern "C" int kvq_kivi_channel_range(const void* x, int64_t stride_b, int64_t s
   if (bits != 4 && bits != 8) return fail(KVQ_ERR_INVALID, "channel range: bits must be 4 or 8");
   if (((uintptr_t)x % 4) || stride_b % 2 || stride_h % 2 || stride_s % 2)
     return fail(KVQ_ERR_UNSUPPORTED, "channel range: rows must be 4-byte aligned");
-  if (!(q_hi == 0.f || (q_lo >= 0.f && q_lo < q_hi && q_hi < 1.f)))
-    return fail(KVQ_ERR_INVALID, "channel range: quantile levels must lie in [0, 1)");
+  // (a percentile just below 100 or above 50 rounds to the level 1 or to equal levels)
+  if (!(q_hi == 0.f || (q_lo >= 0.f && q_lo <= q_hi && q_hi <= 1.f)))
+    return fail(KVQ_ERR_INVALID, "channel range: quantile levels must lie in [0, 1]");
   if (batch * heads == 0) return KVQ_OK;
   RangeArgs a{};
   a.x = reinterpret_cast<const half_t*>(x);

@@ -34,6 +34,19 @@ def test_channel_range_bitexact(shape, pct, bits):
     assert torch.equal(s.cpu(), rs) and torch.equal(z.cpu(), rz)
 
 
+@pytest.mark.parametrize("pct", [99.999999, 50.000001])
+@pytest.mark.parametrize("n", [1, 2, 301, 9000])
+def test_channel_range_rounded_levels(n, pct):
+    """Percentiles whose fp32 levels are 1, or equal: the ranks are still torch.quantile's."""
+    from llm_kvcache_quantization_amd.cache import kivi_channel_params
+    from oracle import quant as OQ
+
+    k = _k(1, 2, n, seed=n)
+    _, rs, rz = OQ.quantize_asymmetric_per_channel(k, 4, pct)
+    s, z = kivi_channel_params(k.cuda(), 4, pct)
+    assert torch.equal(s.cpu(), rs) and torch.equal(z.cpu(), rz)
+
+
 @pytest.mark.parametrize("pct", [100.0, 99.9])
 def test_channel_range_strides(pct):
     from llm_kvcache_quantization_amd.cache import kivi_channel_params
