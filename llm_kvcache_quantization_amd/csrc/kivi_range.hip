@@ -34,6 +34,7 @@ struct RangeArgs {
   const half_t* x;
   int64_t sb, sh, ss;
   int H, S, units;  // units = B * H
+  int first;        // the launch's first unit (launch_range)
   float qmin, span;
   int r[4];         // ranks: lower tail floor / ceil, upper tail floor / ceil
   float wl, wh;
@@ -77,7 +78,7 @@ __device__ __forceinline__ void store_range(const RangeArgs& a, int64_t at, floa
 template <bool PCT, RowLoad LD>
 __global__ __launch_bounds__(1024) void kivi_range_kernel(RangeArgs a) {
   // 128 consecutive work-groups: 8 units (one an XCD) x 16 channel slices
-  const int slice = (blockIdx.x >> 3) & 15, unit = (blockIdx.x & 7) + 8 * (blockIdx.x >> 7);
+  const int slice = (blockIdx.x >> 3) & 15, unit = a.first + (blockIdx.x & 7) + 8 * (blockIdx.x >> 7);
   if (unit >= a.units) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int waves = blockDim.x >> 6, span = kRows * blockDim.x;
@@ -267,14 +268,20 @@ int range_splits(int64_t units, int tokens) {
   return (int)(fill < most ? fill : most);
 }
 
+// A launch has fewer than 2^32 threads, and a unit is 16 work-groups of up to 1024.
+constexpr int kLaunchUnits = 1 << 17;
+
 template <bool PCT>
-void launch_range(const RangeArgs& a, bool al16, hipStream_t st) {
-  const dim3 grid((unsigned)((a.units + 7) / 8 * 128));
+void launch_range(RangeArgs a, bool al16, hipStream_t st) {
   // 4 waves hold 2048 rows, 16 hold 8192; the percentiles' 64 selects want 16 waves at any length
   // (32 units of 333 tokens: 16.8 us with 4 waves and shuffled scans, 11.1 us)
   const dim3 block(!PCT && a.S <= kRows * 256 ? 256 : 1024);
-  if (al16) hipLaunchKernelGGL((kivi_range_kernel<PCT, kCached>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((kivi_range_kernel<PCT, kDwords>), grid, block, 0, st, a);
+  for (a.first = 0; a.first < a.units; a.first += kLaunchUnits) {
+    const int n = a.units - a.first < kLaunchUnits ? a.units - a.first : kLaunchUnits;
+    const dim3 grid((unsigned)((n + 7) / 8 * 128));
+    if (al16) hipLaunchKernelGGL((kivi_range_kernel<PCT, kCached>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((kivi_range_kernel<PCT, kDwords>), grid, block, 0, st, a);
+  }
 }
 
 }  // namespace
@@ -285,7 +292,7 @@ using namespace kvq;
 
 extern "C" int64_t kvq_kivi_range_scratch_bytes(int32_t batch, int32_t heads, int32_t tokens, float q_hi) {
   const int64_t units = batch > 0 && heads > 0 ? (int64_t)batch * heads : 0;
-  const int n = q_hi == 0.f && units <= (1 << 20) ? range_splits(units, tokens) : 0;
+  const int n = q_hi == 0.f ? range_splits(units, tokens) : 0;
   return n > 1 ? units * n * 128 * (int64_t)sizeof(uint32_t) : 0;
 }
 
@@ -294,7 +301,7 @@ extern "C" int kvq_kivi_channel_range(const void* x, int64_t stride_b, int64_t s
                                       float q_hi, float* scale, float* zero_point, void* scratch,
                                       int64_t scratch_bytes, kvq_stream_t stream) {
   if (!x || !scale || !zero_point) return fail(KVQ_ERR_INVALID, "channel range: NULL pointer");
-  if (batch < 0 || heads < 0 || tokens <= 0 || (int64_t)batch * heads > (1 << 20))
+  if (batch < 0 || heads < 0 || tokens <= 0 || (int64_t)batch * heads > (1 << 30))
     return fail(KVQ_ERR_INVALID, "channel range: bad shape");
   if (bits != 4 && bits != 8) return fail(KVQ_ERR_INVALID, "channel range: bits must be 4 or 8");
   if (((uintptr_t)x % 4) || stride_b % 2 || stride_h % 2 || stride_s % 2)

@@ -47,6 +47,19 @@ def test_channel_range_rounded_levels(n, pct):
     assert torch.equal(s.cpu(), rs) and torch.equal(z.cpu(), rz)
 
 
+@pytest.mark.parametrize("pct", [100.0, 99.0])
+def test_channel_range_many_units(pct):
+    """More (b, head) units than one launch holds (2^18 x 16 work-groups of 1024 threads)."""
+    from llm_kvcache_quantization_amd.cache import kivi_channel_params
+
+    B, H, S = (1 << 15) + 3, 9, 2
+    k = torch.randn(B, H, S, 128, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda").half()
+    s, z = kivi_channel_params(k, 8, pct)
+    sel = [0, 7, 14563, 14564, 29127, B - 1]  # around the launches' boundaries at 2^17 and 2^18 units
+    rs, rz = kivi_channel_params(k[sel].cpu(), 8, pct)
+    assert torch.equal(s[sel].cpu(), rs) and torch.equal(z[sel].cpu(), rz)
+
+
 @pytest.mark.parametrize("pct", [100.0, 99.9])
 def test_channel_range_strides(pct):
     from llm_kvcache_quantization_amd.cache import kivi_channel_params
