@@ -1444,16 +1444,14 @@ class _KiviFamily(_EngineBase):
             if layer_id == 0:
                 self._oor_step_counter += 1
             oor_check = self._oor_step_counter % self._oor_check_interval == 0
+        # a prompt's K parameters are the cache's only once the append has accepted K and V (its
+        # status word below): a rejected prompt leaves none, and the next one is a prefill again
+        ks, kz = self._k_scale[layer_id], self._k_zp[layer_id]
         if prefill:
-            # a NaN / Inf is found by the append's status word below, which then undoes this
-            before = self._k_scale[layer_id], self._k_zp[layer_id]
-            self._k_scale[layer_id], self._k_zp[layer_id] = kivi_channel_params(k, kb, self.k_percentile)
-            self._k_scale_initialized[layer_id] = True
-        if kb != 16:
-            ks = self._k_scale[layer_id]
-            if tuple(ks.shape) != (B, H, D):
-                raise ValueError(f"Inconsistent decode K scale/zp shape for layer {layer_id}: "
-                                 f"expected {(B, H, D)}, got {tuple(ks.shape)}")
+            ks, kz = kivi_channel_params(k, kb, self.k_percentile)
+        if kb != 16 and tuple(ks.shape) != (B, H, D):
+            raise ValueError(f"Inconsistent decode K scale/zp shape for layer {layer_id}: "
+                             f"expected {(B, H, D)}, got {tuple(ks.shape)}")
         # the status words (NaN flags, K range count) cost a host sync: read at prefill with
         # check_numerics, and on the decode steps the range check selects
         status = self._status_buf(k.device) if (self.check_numerics and prefill) or oor_check else None
@@ -1466,7 +1464,6 @@ class _KiviFamily(_EngineBase):
         else:
             pk = C.AppendParams()
             _fill_append(pk, _kivi_format(kb), ksx, 32, self._k_cache[layer_id], old, sp)
-            ks, kz = self._k_scale[layer_id], self._k_zp[layer_id]
             pk.static_scale, pk.static_zp = ks.data_ptr(), kz.data_ptr()
             pk.static_scale_dtype = C.KVQ_DTYPE_F32
             pk.static_stride_b, pk.static_stride_h, pk.static_stride_g = ks.stride()
@@ -1487,8 +1484,6 @@ class _KiviFamily(_EngineBase):
         if status is not None:
             st = self._read_status()
             if prefill and st[0] & 1:
-                self._k_scale[layer_id], self._k_zp[layer_id] = before
-                self._k_scale_initialized[layer_id] = False
                 raise ValueError("quantize_asymmetric: input contains NaN or Inf")
             if st[0] & 1 or st[2] & 1:
                 raise ValueError(f"KIVI append: {'K' if st[0] & 1 else 'V'} input contains NaN or Inf "
@@ -1500,6 +1495,9 @@ class _KiviFamily(_EngineBase):
                     f"ENG-041: KIVI decode K clipping at layer {layer_id}: {ratio:.1%} of values exceed "
                     f"prefill-computed scale range [{lo}, {hi}]. Decode token magnitudes may have drifted "
                     "beyond prefill calibration. Attention accuracy may degrade.", RuntimeWarning)
+        if prefill:
+            self._k_scale[layer_id], self._k_zp[layer_id] = ks, kz
+            self._k_scale_initialized[layer_id] = True
         self._layer_seq_lens[layer_id] = old + S
         self._seq_len = max(self._layer_seq_lens)
 

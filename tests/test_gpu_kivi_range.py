@@ -108,6 +108,26 @@ def test_prefill_rejects_nan_and_keeps_no_parameters():
     assert cache.get_seq_len() == 40
 
 
+@pytest.mark.parametrize("side", ["k", "v"])
+def test_rejected_prefill_then_another_prompt(side):
+    """Without clear(): the next prompt is a prefill again, with parameters of its own, and checked."""
+    from llm_kvcache_quantization_amd import KIVIStyleKVCache
+
+    k = _k(1, 2, 40, 3).cuda()
+    bad = k.clone()
+    bad[0, 1, 20, 100] = float("inf")
+    k2, v2 = _k(1, 2, 33, 4).cuda() * 0.25, _k(1, 2, 33, 5).cuda()
+    cache, fresh = (KIVIStyleKVCache(1, quant_bits=4) for _ in range(2))
+    for _ in range(2):  # the second rejection comes from the same check
+        with pytest.raises(ValueError, match="NaN or Inf"):
+            cache.append(0, *((bad, k) if side == "k" else (k, bad)))
+        assert cache.get_seq_len() == 0
+    cache.append(0, k2, v2)
+    fresh.append(0, k2, v2)
+    for a, b in zip(cache.get_kivi_tensors(0), fresh.get_kivi_tensors(0)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("shape", [(1, 1, 8193), (2, 32, 1024), (3, 5, 4370), (1, 2, 33000), (16, 9, 1100)], ids=str)
 def test_split_range_equals_one_launch(shape):
     """Long prompts in two launches over splits of the tokens: the same bits as the single launch
