@@ -119,6 +119,7 @@ class _EngineBase:
         # the decode step's per-layer status rows and the appends not read yet
         self._step_status: Optional[Tensor] = None
         self._step_seen: List[List[int]] = []
+        self._step_unread = False  # a row was handed to a step since the last read
         self._step_pending: List[tuple] = []
         self._step_seq_len0 = 0
         # per layer: the LayerStep over the layer's buffers and the fused append's parameter
@@ -225,6 +226,7 @@ class _EngineBase:
             self._flush_step_status()
         if not self._step_pending:  # the first append of a step: its length before the step
             self._step_seq_len0 = self._seq_len
+        self._step_unread = True
         return buf.data_ptr() + 16 * layer_id
 
     def _defer_status(self, layer_id: int, n_elem: int, kind: str, qrange: str,
@@ -247,7 +249,9 @@ class _EngineBase:
             return
         self._step_pending = []
         rows, seen = self._step_status.cpu().tolist(), self._step_seen
-        self._step_seen = rows
+        self._step_seen, self._step_unread = rows, False
+        if any(r[0] or r[2] for r in rows):  # (of a row not pending too: its step raised)
+            self._clear_step_status()
         bad = None
         for layer_id, n_elem, kind, qrange, clip_warn in pending:
             st = _since(rows[layer_id], seen[layer_id])
@@ -256,18 +260,22 @@ class _EngineBase:
             if clip_warn:
                 self._clip_warnings(layer_id, n_elem, qrange, st)
         if bad is not None:
-            self._discard_step_status(True)
             for layer_id, *_ in pending:
                 self._layer_seq_lens[layer_id] -= 1
             self._seq_len = self._step_seq_len0
             raise ValueError(f"{bad[0]} append: {bad[1]} input contains NaN or Inf — refusing "
                              "to quantize corrupt data")
 
-    def _discard_step_status(self, unread: bool = False) -> None:
-        """Drops the pending rows; clears the buffer if it holds counts not read (or `unread`)."""
-        if (self._step_pending or unread) and self._step_status is not None:
-            self._step_status.zero_()
-            self._step_seen = [[0] * 4 for _ in range(self.num_layers)]
+    def _clear_step_status(self) -> None:
+        self._step_status.zero_()
+        self._step_seen = [[0] * 4 for _ in range(self.num_layers)]
+        self._step_unread = False
+
+    def _discard_step_status(self) -> None:
+        """Drops the pending rows and every count not read, also of a step that raised after its
+        append was enqueued."""
+        if self._step_unread:
+            self._clear_step_status()
         self._step_pending = []
 
     def _read_status(self) -> List[int]:
