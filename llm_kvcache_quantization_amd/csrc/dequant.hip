@@ -130,14 +130,21 @@ void go(const DeqSide& k, const DeqSide& v, int B, int H, int n, hipStream_t st)
   hipLaunchKernelGGL((dequant_kernel<FK, FV, R>), dim3((unsigned)gx, 2), dim3(kDeqWaves * 64), 0, st, k, v,
                      B, H, n);
 }
-template <int FK>
-void go_v(const DeqSide& k, const DeqSide& v, int B, int H, int n, hipStream_t st) {
-  switch (v.codes ? v.fmt : FK) {
-    case KVQ_FMT_INT8_SYM: go<FK, KVQ_FMT_INT8_SYM>(k, v, B, H, n, st); break;
-    case KVQ_FMT_INT4_SYM: go<FK, KVQ_FMT_INT4_SYM>(k, v, B, H, n, st); break;
-    case KVQ_FMT_INT8_KIVI: go<FK, KVQ_FMT_INT8_KIVI>(k, v, B, H, n, st); break;
-    default: go<FK, KVQ_FMT_INT4_KIVI>(k, v, B, H, n, st); break;
-  }
+
+// the launch of a pair of formats (those the engines form), or nullptr
+using Launch = void (*)(const DeqSide&, const DeqSide&, int, int, int, hipStream_t);
+Launch pick(int fk, int fv) {
+#define KVQ_DEQ(A, B) if (fk == A && fv == B) return go<A, B>
+  KVQ_DEQ(KVQ_FMT_INT8_SYM, KVQ_FMT_INT8_SYM);
+  KVQ_DEQ(KVQ_FMT_INT4_SYM, KVQ_FMT_INT4_SYM);
+  KVQ_DEQ(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT4_KIVI);
+  KVQ_DEQ(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT8_KIVI);
+  KVQ_DEQ(KVQ_FMT_INT8_KIVI, KVQ_FMT_INT4_KIVI);
+  KVQ_DEQ(KVQ_FMT_INT8_KIVI, KVQ_FMT_INT8_KIVI);
+  KVQ_DEQ(KVQ_FMT_INT8_SYM, KVQ_FMT_INT4_KIVI);
+  KVQ_DEQ(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT8_SYM);
+#undef KVQ_DEQ
+  return nullptr;
 }
 
 int fill_side(const kvq_kv_view* x, int32_t fmt, int32_t gs, void* out, DeqSide& d, const char* name) {
@@ -185,14 +192,12 @@ extern "C" int kvq_dequant(const kvq_kv_view* k, int32_t k_format, int32_t k_gro
   if (rc) return rc;
   if ((rc = fill_side(v, v_format, v_group, v_out, dv, "v"))) return rc;
   if ((int64_t)batch * heads * tokens > (1 << 30)) return fail(KVQ_ERR_UNSUPPORTED, "dequant: too many rows");
-  if ((int64_t)batch * heads * tokens == 0 || (!k && !v)) return KVQ_OK;
+  if (!k && !v) return KVQ_OK;
+  const Launch launch = pick(dk.codes ? dk.fmt : dv.fmt, dv.codes ? dv.fmt : dk.fmt);
+  if (!launch) return fail(KVQ_ERR_UNSUPPORTED, "dequant: no kernel for this pair of formats");
+  if ((int64_t)batch * heads * tokens == 0) return KVQ_OK;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  switch (dk.codes ? dk.fmt : dv.fmt) {
-    case KVQ_FMT_INT8_SYM: go_v<KVQ_FMT_INT8_SYM>(dk, dv, batch, heads, tokens, st); break;
-    case KVQ_FMT_INT4_SYM: go_v<KVQ_FMT_INT4_SYM>(dk, dv, batch, heads, tokens, st); break;
-    case KVQ_FMT_INT8_KIVI: go_v<KVQ_FMT_INT8_KIVI>(dk, dv, batch, heads, tokens, st); break;
-    default: go_v<KVQ_FMT_INT4_KIVI>(dk, dv, batch, heads, tokens, st); break;
-  }
+  launch(dk, dv, batch, heads, tokens, st);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? KVQ_OK : fail(KVQ_ERR_LAUNCH, std::string("launch: ") + hipGetErrorString(e));
 }

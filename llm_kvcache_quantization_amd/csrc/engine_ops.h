@@ -25,7 +25,9 @@ int kvq_kivi_channel_range(const void* x, int64_t stride_b, int64_t stride_h, in
 // Dequantised fp16 rows [B, H, tokens, 128] (dense) of K and V views (either NULL: left out) in
 // the formats INT8_SYM / INT4_SYM (scale views as kvq_decode_attn takes them, any strides, in
 // groups of k_group / v_group) and INT8_KIVI / INT4_KIVI (fp32 scale / zero-point per channel,
-// scale_stride_g 1, or per token, scale_stride_g 0): get_kv of the engines.
+// scale_stride_g 1, or per token, scale_stride_g 0): get_kv of the engines.  The pairs are those the
+// engines form: both sides INT8_SYM or both INT4_SYM, any two KIVI formats, and INT8_SYM with
+// INT4_KIVI.
 int kvq_dequant(const kvq_kv_view* k, int32_t k_format, int32_t k_group, void* k_out, const kvq_kv_view* v,
                 int32_t v_format, int32_t v_group, void* v_out, int32_t batch, int32_t heads,
                 int32_t tokens, kvq_stream_t stream);
