@@ -191,6 +191,9 @@ def lib() -> ctypes.CDLL:
         pv = ctypes.POINTER(KvView)
         L.kvq_dequant.argtypes = [pv, c_i32, c_i32, c_vp, pv, c_i32, c_i32, c_vp, c_i32, c_i32, c_i32, c_vp]
         L.kvq_dequant.restype = c_i32
+        L.kvq_append_plan.argtypes = [ctypes.POINTER(AppendParams), ctypes.POINTER(AppendParams),
+                                      ctypes.POINTER(c_i32)]
+        L.kvq_append_plan.restype = c_i32
         ver = L.kvq_abi_version()
         if ver != ABI_VERSION:
             raise ImportError(f"{LIB_PATH} has ABI {ver}, this package needs {ABI_VERSION}; rebuild it")

@@ -28,10 +28,25 @@ struct BulkSide {
   float w, bw;
 };
 
-// Launches the tile kernel for the append of k and v if it takes both (else false, nothing
-// enqueued).  The caller has validated both sides (fill_dev); a side's group rescue has its
-// threshold selected in its scratch, or with `local` (at most kRescueMax scales) every work-group
-// finds it.
-bool append_bulk(const AppendDev& k, const AppendDev& v, hipStream_t st, bool local);
+// A launch of the tile kernel
+struct BulkPlan {
+  BulkSide ks, vs;
+  int ck, cv;       // the sides' formats, TILE32 apart from rows
+  int tok;          // tokens a wave takes at a time
+  int waves;        // a work-group
+  unsigned groups;  // work-groups a side
+};
+
+// Whether the tile kernel takes the append of k and v, and how.  It takes what the engines hand over:
+// both sides INT8_SYM or both INT4_SYM, any two KIVI formats, INT8_SYM with INT4_KIVI, INT4_ASYM or
+// INT8_SYM K with TILE32 V, and any of the former's sides alone, from kBulkMinTokens tokens on, with
+// 16-byte aligned rows, code rows aligned to a lane's store and percentiles within the two largest
+// (smallest) values of a group.  Every other append is the row kernel's at any length: INT4_ASYM in
+// token rows on both sides or either INT4_ASYM side alone, and FP16 rows beside a quantized side (the
+// engines copy those with torch and append the other side alone).  The caller has validated both
+// sides (fill_dev); a side's group rescue has its threshold selected in its scratch, or with `local`
+// (at most kRescueMax scales) every work-group finds it.
+bool bulk_plan(const AppendDev& k, const AppendDev& v, bool local, BulkPlan& p);
+void append_bulk(const AppendDev& k, const AppendDev& v, const BulkPlan& p, hipStream_t st);
 
 }  // namespace kvq

@@ -564,10 +564,28 @@ bool side_ok(const AppendDev& d, BulkSide& s) {
 }
 
 template <int FK, int FV, int NT, bool KT = false, bool VT = false>
-void go(const AppendDev& k, const AppendDev& v, const BulkSide& ks, const BulkSide& vs, unsigned gx,
-        int waves, hipStream_t st) {
-  hipLaunchKernelGGL((append_bulk_kernel<FK, FV, NT, KT, VT>), dim3(gx, 2), dim3(waves * 64), 0, st, k, v,
-                     ks, vs);
+void go(const AppendDev& k, const AppendDev& v, const BulkPlan& p, hipStream_t st) {
+  hipLaunchKernelGGL((append_bulk_kernel<FK, FV, NT, KT, VT>), dim3(p.groups, 2), dim3(p.waves * 64), 0, st, k,
+                     v, p.ks, p.vs);
+}
+
+// the launch of a pair of side codes with tok tokens a wave, or nullptr
+using Launch = void (*)(const AppendDev&, const AppendDev&, const BulkPlan&, hipStream_t);
+Launch pick(int ck, int cv, int tok) {
+#define KVQ_BULK(A, B) \
+  if (ck == A && cv == B) return tok == 32 ? go<A, B, 8> : tok == 16 ? go<A, B, 4> : go<A, B, 2>
+  KVQ_BULK(KVQ_FMT_INT8_SYM, KVQ_FMT_INT8_SYM);
+  KVQ_BULK(KVQ_FMT_INT4_SYM, KVQ_FMT_INT4_SYM);
+  KVQ_BULK(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT4_KIVI);
+  KVQ_BULK(KVQ_FMT_INT8_KIVI, KVQ_FMT_INT8_KIVI);
+  KVQ_BULK(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT8_KIVI);
+  KVQ_BULK(KVQ_FMT_INT8_KIVI, KVQ_FMT_INT4_KIVI);
+  KVQ_BULK(KVQ_FMT_INT8_SYM, KVQ_FMT_INT4_KIVI);
+  KVQ_BULK(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT8_SYM);
+#undef KVQ_BULK
+  if (ck == KVQ_FMT_INT4_ASYM && cv == kTileAsym) return go<KVQ_FMT_INT4_ASYM, KVQ_FMT_INT4_ASYM, 8, false, true>;
+  if (ck == KVQ_FMT_INT8_SYM && cv == kTileAsym) return go<KVQ_FMT_INT8_SYM, KVQ_FMT_INT4_ASYM, 8, false, true>;
+  return nullptr;
 }
 
 int64_t tiles_of(const AppendDev& d, int tok) {
@@ -578,54 +596,33 @@ int64_t tiles_of(const AppendDev& d, int tok) {
 
 }  // namespace
 
-bool append_bulk(const AppendDev& k, const AppendDev& v, hipStream_t st, bool local) {
-  BulkSide ks, vs;
-  if (!side_ok(k, ks) || !side_ok(v, vs)) return false;
-  const int s_new = k.valid ? k.S : v.S;
-  if (s_new < kBulkMinTokens) return false;
-  ks.local = local && needs_threshold(k);
-  vs.local = local && needs_threshold(v);
+bool bulk_plan(const AppendDev& k, const AppendDev& v, bool local, BulkPlan& p) {
+  if (!side_ok(k, p.ks) || !side_ok(v, p.vs)) return false;
+  if ((k.valid ? k.S : v.S) < kBulkMinTokens) return false;
+  p.ks.local = local && needs_threshold(k);
+  p.vs.local = local && needs_threshold(v);
   // a missing side runs as the other one's format (its work-groups exit at once)
-  const int ck = k.valid ? side_code(k) : side_code(v), cv = v.valid ? side_code(v) : side_code(k);
+  p.ck = k.valid ? side_code(k) : side_code(v);
+  p.cv = v.valid ? side_code(v) : side_code(k);
   // 32 tokens a wave where that gives every SIMD a few waves, fewer in shorter prompts
   const int64_t t32 = tiles_of(k, 32) > tiles_of(v, 32) ? tiles_of(k, 32) : tiles_of(v, 32);
-  const bool tiled = ck == kTileAsym || cv == kTileAsym;
-  const int tok = tiled || t32 >= kBulkTiles32 ? 32 : t32 >= kBulkTiles16 ? 16 : 8;
-  const int64_t tiles = tiles_of(k, tok) > tiles_of(v, tok) ? tiles_of(k, tok) : tiles_of(v, tok);
+  const bool tiled = p.ck == kTileAsym || p.cv == kTileAsym;
+  p.tok = tiled || t32 >= kBulkTiles32 ? 32 : t32 >= kBulkTiles16 ? 16 : 8;
+  const int64_t tiles = tiles_of(k, p.tok) > tiles_of(v, p.tok) ? tiles_of(k, p.tok) : tiles_of(v, p.tok);
   if (tiles > ((int64_t)1 << 30)) return false;
   // every work-group that clipped adds to one status word, and such atomics queue (about 10 ns
   // each): 8 waves a work-group where that counts and the tiles fill the SIMDs, else 4
-  const int waves = local || (tiles >= kBulkWideFrom && tiles < kBulkWideTo) ? 8 : 4;
-  int64_t gx = (tiles + waves - 1) / waves;
+  p.waves = local || (tiles >= kBulkWideFrom && tiles < kBulkWideTo) ? 8 : 4;
+  int64_t gx = (tiles + p.waves - 1) / p.waves;
   // at most 64 tiles a wave (its redo mask)
-  const int64_t least = (tiles + 64 * waves - 1) / (64 * waves), most = kBulkWaveSlots / waves;
+  const int64_t least = (tiles + 64 * p.waves - 1) / (64 * p.waves), most = kBulkWaveSlots / p.waves;
   if (gx > most) gx = most > least ? most : least;
-  const unsigned g = (unsigned)gx;
-#define KVQ_BULK(A, B)                                   \
-  if (ck == A && cv == B) {                              \
-    if (tok == 32) go<A, B, 8>(k, v, ks, vs, g, waves, st);      \
-    else if (tok == 16) go<A, B, 4>(k, v, ks, vs, g, waves, st); \
-    else go<A, B, 2>(k, v, ks, vs, g, waves, st);                \
-    return true;                                         \
-  }
-  KVQ_BULK(KVQ_FMT_INT8_SYM, KVQ_FMT_INT8_SYM)
-  KVQ_BULK(KVQ_FMT_INT4_SYM, KVQ_FMT_INT4_SYM)
-  KVQ_BULK(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT4_KIVI)
-  KVQ_BULK(KVQ_FMT_INT8_KIVI, KVQ_FMT_INT8_KIVI)
-  KVQ_BULK(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT8_KIVI)
-  KVQ_BULK(KVQ_FMT_INT8_KIVI, KVQ_FMT_INT4_KIVI)
-  KVQ_BULK(KVQ_FMT_INT8_SYM, KVQ_FMT_INT4_KIVI)
-  KVQ_BULK(KVQ_FMT_INT4_KIVI, KVQ_FMT_INT8_SYM)
-#undef KVQ_BULK
-  if (ck == KVQ_FMT_INT4_ASYM && cv == kTileAsym) {
-    go<KVQ_FMT_INT4_ASYM, KVQ_FMT_INT4_ASYM, 8, false, true>(k, v, ks, vs, g, waves, st);
-    return true;
-  }
-  if (ck == KVQ_FMT_INT8_SYM && cv == kTileAsym) {
-    go<KVQ_FMT_INT8_SYM, KVQ_FMT_INT4_ASYM, 8, false, true>(k, v, ks, vs, g, waves, st);
-    return true;
-  }
-  return false;
+  p.groups = (unsigned)gx;
+  return pick(p.ck, p.cv, p.tok) != nullptr;
+}
+
+void append_bulk(const AppendDev& k, const AppendDev& v, const BulkPlan& p, hipStream_t st) {
+  pick(p.ck, p.cv, p.tok)(k, v, p, st);
 }
 
 }  // namespace kvq

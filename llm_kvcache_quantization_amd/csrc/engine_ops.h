@@ -32,6 +32,11 @@ int kvq_dequant(const kvq_kv_view* k, int32_t k_format, int32_t k_group, void* k
                 int32_t v_format, int32_t v_group, void* v_out, int32_t batch, int32_t heads,
                 int32_t tokens, kvq_stream_t stream);
 
+// The launch kvq_quant_append makes for k and v (host only: nothing is enqueued).  plan[0]: 0 nothing
+// to append, 1 the row kernel, 2 the tile kernel; plan[1] tokens of a head a wave takes at a time;
+// plan[2] waves a work-group; plan[3] work-groups a side.
+int kvq_append_plan(const kvq_append_params* k, const kvq_append_params* v, int32_t* plan);
+
 #ifdef __cplusplus
 }
 #endif

@@ -16,6 +16,7 @@
 #include "append_bulk.h"
 #include "append_row.h"
 #include "append_tile.h"
+#include "engine_ops.h"
 #include "kvq_common.h"
 #include "kvq.h"
 
@@ -167,7 +168,7 @@ __device__ float sorted_quantile(const float* v, int n, float q) {
   return quantile_lerp(v[lo], v[hi], rank - (float)lo);
 }
 
-// rescue: 0 none (or the threshold in a.thr_ptr), 1 one work-group finds the threshold and
+// rescue: 0 none (or the threshold from the select in a.rescue), 1 one work-group finds the threshold and
 // quantizes every row, 2 every work-group finds it (rank counting) and quantizes its own rows
 __device__ __forceinline__ void append_side(const AppendDev& a, int rescue) {
   if (!a.valid) return;
@@ -345,6 +346,30 @@ static int take_scratch(const kvq_append_params* p, AppendDev& d, const char* na
   return KVQ_OK;
 }
 
+// How an append finds the thresholds of its group rescues.  `large`: by the key select, when a side
+// has more than kRescueMax scales.  Else `mode`: 0 there is none, 2 at most kRescueRank scales
+// (decode steps), 1 up to kRescueMax; the tile kernel finds either in every work-group, the row kernel
+// 2 in every work-group and 1 in a single one (4 heads x 103 tokens in groups of 16: 267 us in one
+// work-group, 12 by the tile kernel; 2 x 60: 21.5, 8.8).
+struct RescuePlan {
+  bool large;
+  int mode;
+};
+static RescuePlan rescue_plan(const kvq_append_params* k, const kvq_append_params* v) {
+  const int64_t nk = needs_rescue(k) ? rescue_n(k) : 0, nv = needs_rescue(v) ? rescue_n(v) : 0;
+  const int64_t n = nk > nv ? nk : nv;
+  return RescuePlan{n > kRescueMax, n == 0 || n > kRescueMax ? 0 : n <= kRescueRank ? 2 : 1};
+}
+
+// work-groups a side of the row kernel
+static unsigned row_groups(const AppendDev& k, const AppendDev& v, int rescue) {
+  int64_t rows = 0;
+  if (k.valid) rows = (int64_t)k.B * k.H * k.S;
+  if (v.valid) rows = rows > (int64_t)v.B * v.H * v.S ? rows : (int64_t)v.B * v.H * v.S;
+  const int64_t gx = rescue == 1 ? 1 : (rows + kAppendWaves - 1) / kAppendWaves;
+  return (unsigned)(gx > 65535 ? 65535 : gx);
+}
+
 template <RowLoad LD>
 static void rescue_select(const AppendDev& k, const AppendDev& v, unsigned gx, hipStream_t st) {
   hipLaunchKernelGGL((rescue_hist_kernel<0, LD>), dim3(gx, 2), dim3(256), 0, st, k, v);
@@ -384,35 +409,18 @@ extern "C" int kvq_quant_append(const kvq_append_params* k, const kvq_append_par
   if (rc) return rc;
   if (!dk.valid && !dv.valid) return KVQ_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // the group rescue takes its threshold from one work-group's LDS sort when every side
-  // that needs one has at most kRescueMax scales, else from the key select (scratch)
-  const bool large = (needs_rescue(k) && rescue_n(k) > kRescueMax) ||
-                     (needs_rescue(v) && rescue_n(v) > kRescueMax);
-  if (large) {
+  const RescuePlan r = rescue_plan(k, v);
+  if (r.large) {
     if (needs_rescue(k) && (rc = take_scratch(k, dk, "k"))) return rc;
     if (needs_rescue(v) && (rc = take_scratch(v, dv, "v"))) return rc;
     rescue_large(dk, dv, s);
   }
-  // rescues over at most kRescueMax scales: a prompt's tile kernel finds the threshold in every
-  // work-group (4 heads x 103 tokens in groups of 16: 267 -> 12 us, 2 x 60: 21.5 -> 8.8 us), the
-  // row kernel in every work-group up to kRescueRank scales (decode steps), else in one
-  int rescue = 0;
-  if (!large && (needs_rescue(k) || needs_rescue(v))) {
-    const int64_t nk = needs_rescue(k) ? rescue_n(k) : 0, nv = needs_rescue(v) ? rescue_n(v) : 0;
-    rescue = (nk > nv ? nk : nv) <= kRescueRank ? 2 : 1;
-  }
-  if (append_bulk(dk, dv, s, rescue != 0)) {
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(KVQ_ERR_LAUNCH, std::string("launch: ") + hipGetErrorString(e));
-    return KVQ_OK;
-  }
-  int64_t rows = 0;
-  if (dk.valid) rows = (int64_t)dk.B * dk.H * dk.S;
-  if (dv.valid) rows = rows > (int64_t)dv.B * dv.H * dv.S ? rows : (int64_t)dv.B * dv.H * dv.S;
-  int64_t gx = rescue == 1 ? 1 : (rows + kAppendWaves - 1) / kAppendWaves;
-  if (gx > 65535) gx = 65535;
-  hipLaunchKernelGGL(append_kernel, dim3((unsigned)gx, 2), dim3(kAppendWaves * 64), 0, s, dk, dv,
-                     rescue);
+  BulkPlan plan;
+  if (bulk_plan(dk, dv, r.mode != 0, plan))
+    append_bulk(dk, dv, plan, s);
+  else
+    hipLaunchKernelGGL(append_kernel, dim3(row_groups(dk, dv, r.mode), 2), dim3(kAppendWaves * 64), 0, s, dk, dv,
+                       r.mode);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(KVQ_ERR_LAUNCH, std::string("launch: ") + hipGetErrorString(e));
   return KVQ_OK;
@@ -420,4 +428,26 @@ extern "C" int kvq_quant_append(const kvq_append_params* k, const kvq_append_par
 
 extern "C" int64_t kvq_append_scratch_bytes(const kvq_append_params* p) {
   return (needs_rescue(p) && rescue_n(p) > kRescueMax) ? (int64_t)sizeof(RescueScratch) : 0;
+}
+
+extern "C" int kvq_append_plan(const kvq_append_params* k, const kvq_append_params* v, int32_t* plan) {
+  AppendDev dk, dv;
+  int rc = fill_dev(k, dk, "k");
+  if (rc) return rc;
+  if ((rc = fill_dev(v, dv, "v"))) return rc;
+  for (int i = 0; i < 4; ++i) plan[i] = 0;
+  if (!dk.valid && !dv.valid) return KVQ_OK;
+  const RescuePlan r = rescue_plan(k, v);
+  BulkPlan p;
+  if (bulk_plan(dk, dv, r.mode != 0, p)) {
+    plan[0] = 2;
+    plan[1] = p.tok;
+    plan[2] = p.waves;
+    plan[3] = (int32_t)p.groups;
+  } else {
+    plan[0] = plan[1] = 1;
+    plan[2] = kAppendWaves;
+    plan[3] = (int32_t)row_groups(dk, dv, r.mode);
+  }
+  return KVQ_OK;
 }

@@ -1,10 +1,12 @@
 """The prompt-sized append (csrc/append_bulk.hip) against the row kernel, bit for bit.
 
 Both kernels append the same values: once from dense rows (which the tile kernel takes) and once
-from rows 130 values apart (not 16-byte aligned, so the row kernel quantizes them).  Codes, scales,
-zero-points, outlier values and status words must be equal, also where the tile kernel hands tiles
-back: NaN / Inf rows, zero or infinite scales.  The row kernel itself is pinned to the oracle by
-the append tests of test_gpu_parity.py and test_gpu_kivi_family.py, at sizes that run both."""
+from rows 130 values apart (not 16-byte aligned, so the row kernel quantizes them); the library's
+plan of each call says which kernel ran.  Codes, scales, zero-points, outlier values and status words
+must be equal, also where the tile kernel hands tiles back: NaN / Inf rows, zero or infinite scales.
+The row kernel itself is pinned to the oracle by the append tests of test_gpu_parity.py and
+test_gpu_kivi_family.py: their appends of fewer than 8 tokens, and test_gpu_parity.py's unaligned
+rows."""
 import ctypes
 
 import pytest
@@ -128,9 +130,47 @@ PAIRS = {
 }
 
 # (batch, heads, tokens, write position): fewest tokens, a tile's edges, starts inside a tile, a
-# size whose rescue threshold every work-group finds (1025 to 4096 scales), and enough tiles for
-# 32 tokens a wave in every format
-SIZES = [(1, 2, 8, 0), (2, 3, 31, 5), (1, 1, 33, 31), (3, 2, 64, 32), (2, 8, 4099, 1)]
+# size whose rescue threshold every work-group finds (1025 to 4096 scales), then 1032 and 2064
+# 32-token tiles: 16 and 32 tokens a wave in every row format
+SIZES = [(1, 2, 8, 0), (2, 3, 31, 5), (1, 1, 33, 31), (3, 2, 64, 32), (2, 4, 4099, 1), (2, 8, 4099, 1)]
+
+
+def _plan(pk, pv):
+    """(0 nothing / 1 row kernel / 2 tile kernel, tokens a wave, waves a work-group, work-groups)"""
+    C, L = _lib()
+    out = (ctypes.c_int32 * 4)()
+    C.check(L.kvq_append_plan(*(None if p is None else ctypes.byref(p) for p in (pk, pv)), out))
+    return tuple(out)
+
+
+def _append(name, x, wpos, cap, sides=(0, 1)):
+    """The tensors an append of x[side] (a list of 2) writes, and its plan; sides: those not NULL."""
+    C, L = _lib()
+    ps, wrote, keep = [None, None], [], []
+    for side in sides:
+        fmt, gs, policy = PAIRS[name][side][:3]
+        B, H, S = x[side].shape[:3]
+        g = torch.Generator(device="cuda").manual_seed(99 + side)
+        p, o, kp = _side(C, fmt, gs, B, H, S, wpos, cap, x[side], policy, g, tile=len(PAIRS[name][side]) > 3)
+        ps[side] = p
+        wrote += o
+        keep += kp
+    plan = _plan(*ps)
+    C.check(L.kvq_quant_append(*(None if p is None else ctypes.byref(p) for p in ps),
+                               ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    return wrote, plan
+
+
+def _apart(x, w):
+    """x in rows w values apart."""
+    out = torch.zeros(*x.shape[:3], w, dtype=torch.float16, device="cuda")[..., :D]
+    return out.copy_(x)
+
+
+def _same(a, b, what):
+    for i, j in zip(a, b, strict=True):  # bits: NaN scales of NaN rows included
+        assert torch.equal(i.contiguous().view(torch.uint8), j.contiguous().view(torch.uint8)), (what, i.dtype)
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
@@ -169,6 +209,13 @@ def test_bulk_append_equals_row_kernel(name, size):
             ps.append(p)
             wrote += o
             keep += kp
+        kernel, tok = _plan(*ps)[:2]
+        if route == 0:
+            t32 = B * H * -(-S // 32)
+            tiled = any(len(spec) > 3 for spec in PAIRS[name])
+            assert kernel == 2 and tok == (32 if tiled or t32 >= 2048 else 16 if t32 >= 512 else 8)
+        else:
+            assert kernel == 1
         C.check(L.kvq_quant_append(ctypes.byref(ps[0]), ctypes.byref(ps[1]),
                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
         torch.cuda.synchronize()
@@ -176,3 +223,56 @@ def test_bulk_append_equals_row_kernel(name, size):
     for a, b in zip(*outs):
         # bits: NaN scales of NaN rows included
         assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8)), (name, a.dtype)
+
+
+@pytest.mark.parametrize("name", ["int8_table_odd", "int4_rescue_nan", "asym_odd", "kivi8_odd"])
+def test_tiles_after_a_waves_first(name):
+    """More tiles than waves: those a wave takes second and third, some handed back."""
+    B, H, S, wpos = 2, 8, 33000, 1
+    cap = 33024
+    x = []
+    for side in range(2):
+        v = torch.randn(B, H, S, D, generator=torch.Generator(device="cuda").manual_seed(side), device="cuda").half()
+        v[-1, -1, -5, 100] = float("nan")  # the last tiles are some waves' third
+        v[-1, -1, -70, 3] = float("inf")
+        v[-1, 2, 40, 64] = -float("inf")   # a second one
+        v[0, 1, 3, 9] = float("nan")       # a first one
+        x.append(v)
+    tile, plan = _append(name, x, wpos, cap)
+    assert plan[:2] == (2, 32) and 2 * plan[2] * plan[3] < B * H * 1032
+    row, plan = _append(name, [_apart(v, 130) for v in x], wpos, cap)
+    assert plan[0] == 1
+    _same(tile, row, name)
+
+
+@pytest.mark.parametrize("side", [0, 1])
+@pytest.mark.parametrize("name", ["int8_p999", "int8_table_g16", "int4_rescue_g16", "int4_p999_g16", "kivi4_p999",
+                                  "kivi8", "kivi48", "mixed", "k8_asym", "asym_tile"])
+@pytest.mark.parametrize("size", [(2, 3, 31, 5), (2, 4, 4099, 1)], ids=str)
+def test_one_side(size, name, side):
+    """K or V alone (a cache whose other side is 16-bit): the same bits as beside the other side."""
+    B, H, S, wpos = size
+    cap = -(-(wpos + S) // 32) * 32
+    x = [torch.randn(B, H, S, D, generator=torch.Generator(device="cuda").manual_seed(s), device="cuda").half()
+         for s in (5, 6)]
+    both, _ = _append(name, x, wpos, cap)
+    one, plan = _append(name, x, wpos, cap, sides=(side,))
+    fmt = PAIRS[name][side][0]
+    assert plan[0] == (1 if fmt == A4 else 2)
+    _same(one, both[:len(one)] if side == 0 else both[-len(one):], name)
+
+
+@pytest.mark.parametrize("name", ["int8_p999", "int4_rescue_g16", "asym_tile", "kivi8", "mixed"])
+@pytest.mark.parametrize("size", [(2, 3, 131, 5), (2, 4, 4099, 1)], ids=str)
+def test_strides(size, name):
+    """Rows the tile kernel takes in other layouts: tokens outside the heads, padded rows."""
+    B, H, S, wpos = size
+    cap = -(-(wpos + S) // 32) * 32
+    x = [torch.randn(B, H, S, D, generator=torch.Generator(device="cuda").manual_seed(s), device="cuda").half()
+         for s in (5, 6)]
+    ref, _ = _append(name, [_apart(v, 130) for v in x], wpos, cap)
+    for layout in (lambda v: v.transpose(1, 2).contiguous().transpose(1, 2), lambda v: _apart(v, 136),
+                   lambda v: v.permute(2, 0, 1, 3).contiguous().permute(1, 2, 0, 3)):
+        got, plan = _append(name, [layout(v) for v in x], wpos, cap)
+        assert plan[0] == 2
+        _same(got, ref, name)

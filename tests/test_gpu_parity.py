@@ -151,15 +151,15 @@ def test_append_int4_sym_bitexact(mode, S):
 
 
 @pytest.mark.parametrize("B,H,S,ratio,ties,gs", [
-    (2, 4, 2048, 0.01, False, 32),    # 65,536 scales: the radix-select path
+    (2, 4, 2048, 0.01, False, 32),    # 65,536 scales: the key select
     (1, 2, 600, 0.3, True, 32),       # 4,800 scales, many equal (ties at the threshold)
     (4, 2, 4096, 0.001, False, 32),   # 131,072 scales, a threshold in the far tail
-    (2, 2, 256, 0.05, False, 32),     # 4,096 scales: the one-work-group sort path
+    (2, 2, 256, 0.05, False, 32),     # 4,096 scales, the most the tile kernel's work-groups find
     (40, 8, 1, 0.01, True, 32),       # 1,280 scales: the one-work-group walk from the top
     (8, 4, 1, 0.01, False, 32),       # a decode step (128 scales): rank counting
     (16, 4, 1, 0.01, True, 32),       # 64 rows, ties
     (8, 4, 1, 0.1, False, 32),        # 13 ranks below the top
-    (4, 2, 16, 0.05, True, 32),       # 512 scales, 26 ranks below the top, ties
+    (4, 2, 16, 0.05, True, 32),       # the tile kernel: 512 scales, 26 ranks below the top, ties
     (8, 4, 1, 0.01, False, 16),       # config 3's decode step at group 16 (256 scales)
     (3, 3, 1, 0.2, False, 128),       # 9 rows and 9 scales (not a multiple of 4)
     (32, 8, 1, 0.01, True, 32),       # 1,024 scales: the most that are rank-counted
@@ -168,9 +168,29 @@ def test_append_int4_sym_bitexact(mode, S):
 ])
 def test_append_int4_rescue_large_bitexact(B, H, S, ratio, ties, gs):
     """INT4 group outlier rescue over the dynamic scales of an append: the torch.quantile
-    threshold (int4_cache.py:384-390) by the radix select in the scratch buffer (more than
-    4096 scales), one work-group's LDS sort or walk from the top (1025-4096), or rank
-    counting in every work-group (at most 1024), codes and scales bit-exact."""
+    threshold (int4_cache.py:384-390) by the key select in the scratch buffer (more than 4096
+    scales), in every work-group of the tile kernel (8 tokens and more), by the row kernel's one
+    work-group from the top (1025-4096), or by rank counting in its every work-group (at most
+    1024), codes and scales bit-exact."""
+    _rescue_bitexact(B, H, S, ratio, ties, gs)
+
+
+@pytest.mark.parametrize("B,H,S,ratio,ties,gs", [
+    (2, 2, 256, 0.05, False, 32),     # 4,096 scales: one work-group's sort, nothing to pad
+    (1, 3, 130, 0.4, True, 32),       # 1,560 scales, padded to 2,048, ties
+    (64, 8, 1, 0.3, False, 32),       # a wide decode step: 2,048 scales
+    (2, 2, 200, 0.005, True, 32),     # 3,200 scales: its walk from the top
+    (2, 3, 60, 0.2, False, 32),       # 1,440 scales
+    (4, 2, 16, 0.05, True, 32),       # 512: every work-group
+    (2, 3, 400, 0.02, False, 16),     # 19,200: the select over rows aligned to 4 bytes
+])
+def test_append_int4_rescue_row_kernel_bitexact(B, H, S, ratio, ties, gs):
+    """The same threshold where the row kernel quantizes: rows 130 values apart are not 16-byte
+    aligned, whatever their number."""
+    _rescue_bitexact(B, H, S, ratio, ties, gs, apart=130)
+
+
+def _rescue_bitexact(B, H, S, ratio, ties, gs, apart=128):
     K = _lib()
     from llm_kvcache_quantization_amd import _capi as C
 
@@ -191,7 +211,8 @@ def test_append_int4_rescue_large_bitexact(B, H, S, ratio, ties, gs):
     p.static_scale, p.rescue_quantile = 1, float(torch.tensor(1.0 - ratio, dtype=torch.float32))
     n = B * H * S * (D // gs)
     assert (C.lib().kvq_append_scratch_bytes(ctypes.byref(p)) > 0) == (n > 4096)
-    cache.append(0, k.to(DEV), v.to(DEV))
+    kd, vd = (torch.zeros(B, H, S, apart, dtype=torch.float16, device=DEV)[..., :D].copy_(x) for x in (k, v))
+    cache.append(0, kd, vd)
     kp, vp, ks, vs = cache.get_int4_tensors(0)
     for x, stt, p_gpu, s_gpu, tag in ((k, st, kp, ks, "k"), (v, st * 0.8, vp, vs, "v")):
         ref_q, ref_s = OQ.int4_cache_quantize(x, stt, gs, outlier_rescue_ratio=ratio)
