@@ -14,10 +14,16 @@ constexpr int kBulkMinTokens = 8;
 // 256 tiles (INT8, 2 x 4096 tokens) 5.4 / 5.8 / 7.9, 1024 (KIVI INT4, 4 x 8191) 21.2 / 12.5 / 12.5,
 // 1504 (INT4, 8 x 6001) 14.6 / 13.2 / 14.3.
 constexpr int kBulkTiles32 = 2048, kBulkTiles16 = 512;
-// tiles for which a work-group has 8 waves instead of 4 (INT4 with rescued groups, whose largest
-// value often counts as clipped, at 8 x 4096 tokens: 15.5 -> 13.0 us; 700 tiles of the mixed cache
-// 6.5 against 7.3 us, 32768 tiles of the asymmetric format 131 against 135 us)
-constexpr int kBulkWideFrom = 2048, kBulkWideTo = 8192;
+// Tiles for which a work-group has 8 waves instead of 4 where a side counts clipped values (a static
+// table and a status word).  A work-group that clipped adds to the side's one status word and such
+// atomics queue (about 10 ns each), so half as many help as long as about every tile clips and has a
+// wave of its own; a count that stays 0 only pays for the coarser grid.  us for 4 / 8 waves, INT8
+// tables that clip half of the values, and tables that clip none: 1056 tiles 9.6 / 8.9 and 7.8 / 8.7,
+// 1504 10.9 / 9.9 and 8.1 / 9.1, 1952 13.2 / 11.4 and 9.5 / 9.2, 3000 18.3 / 14.3 and 12.2 / 12.1, 8128
+// 60.6 / 44.9 and 44.2 / 44.7, 12000 73.0 / 64.6 and 59.0 / 60.3, 14016 72.4 / 69.6 and 67.3 / 68.2,
+// 20000 90.9 / 91.8 and 89.7 / 92.3.  Sides that count nothing keep 4: INT8 with the 99.9 percentile
+// 2112 tiles 20.6 / 23.2, 4096 30.9 / 31.9, 8128 51.2 / 53.2; the mixed cache 2112 22.6 / 26.2.
+constexpr int kBulkWideFrom = 1728, kBulkWideTo = 13000;
 
 // Order statistics of a percentile (ranks and weight, as torch.quantile computes them) and
 // whether a static table has a per-token policy.

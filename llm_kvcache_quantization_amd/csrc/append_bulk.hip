@@ -610,9 +610,10 @@ bool bulk_plan(const AppendDev& k, const AppendDev& v, bool local, BulkPlan& p) 
   p.tok = tiled || t32 >= kBulkTiles32 ? 32 : t32 >= kBulkTiles16 ? 16 : 8;
   const int64_t tiles = tiles_of(k, p.tok) > tiles_of(v, p.tok) ? tiles_of(k, p.tok) : tiles_of(v, p.tok);
   if (tiles > ((int64_t)1 << 30)) return false;
-  // every work-group that clipped adds to one status word, and such atomics queue (about 10 ns
-  // each): 8 waves a work-group where that counts and the tiles fill the SIMDs, else 4
-  p.waves = local || (tiles >= kBulkWideFrom && tiles < kBulkWideTo) ? 8 : 4;
+  const bool counts = (k.valid && k.st && k.status) || (v.valid && v.st && v.status);
+  // (and where every work-group finds the rescue's threshold, among all rows: 4 / 8 waves, 1 x 2 heads
+  // x 60 tokens in groups of 16 9.3 / 8.6 us, 1 x 4 x 250 in groups of 32 25.0 / 18.1)
+  p.waves = local || (counts && tiles >= kBulkWideFrom && tiles < kBulkWideTo) ? 8 : 4;
   int64_t gx = (tiles + p.waves - 1) / p.waves;
   // at most 64 tiles a wave (its redo mask)
   const int64_t least = (tiles + 64 * p.waves - 1) / (64 * p.waves), most = kBulkWaveSlots / p.waves;

@@ -85,3 +85,17 @@ def test_grid_covers_the_tiles():
         tiles = B * H * -(-S // tok)
         assert kernel == TILE and groups * waves * 64 >= tiles
         assert groups <= max(8192 // waves, -(-tiles // (64 * waves)))
+
+
+def test_waves_a_work_group():
+    """8 where a side counts clipped values and the tiles lie in the measured range, else 4."""
+    for S, wide in ((2048, False), (4096, True), (49152, True), (65536, False)):  # 1024, 2048, 12288, 16384 tiles
+        for k, v, counts in ((_side(I8, S=S, table=True), _side(I8, S=S, table=True), True),
+                             (_side(I8, S=S), _side(I8, S=S, table=True), True),
+                             (_side(K4, S=S, table=True), _side(K4, S=S), True),
+                             (_side(I8, S=S, table=True), None, True),
+                             (_side(I8, S=S, table=True, status=False), _side(I8, S=S, table=True, status=False), False),
+                             (_side(I8, S=S), _side(I8, S=S), False), (_side(I8, S=S), _side(K4, S=S), False)):
+            assert _plan(k, v)[2] == (8 if wide and counts else 4), S
+    # a threshold found by every work-group: 8 waves at any size it applies to
+    assert _plan(*(_side(I4, 1, 2, 60, table=True, rescue_quantile=0.99) for _ in range(2)))[2] == 8
