@@ -194,6 +194,8 @@ def lib() -> ctypes.CDLL:
         L.kvq_append_plan.argtypes = [ctypes.POINTER(AppendParams), ctypes.POINTER(AppendParams),
                                       ctypes.POINTER(c_i32)]
         L.kvq_append_plan.restype = c_i32
+        L.kvq_append_division.argtypes = [c_vp, c_vp, c_vp, c_vp, c_i64, c_vp]
+        L.kvq_append_division.restype = c_i32
         ver = L.kvq_abi_version()
         if ver != ABI_VERSION:
             raise ImportError(f"{LIB_PATH} has ABI {ver}, this package needs {ABI_VERSION}; rebuild it")

@@ -20,6 +20,7 @@
 // [2^-30, 2^30], are left to the row quantizer after the wave's other tiles.
 #include "append_bulk.h"
 #include "append_tile.h"
+#include "engine_ops.h"
 
 #pragma clang fp contract(off)
 
@@ -73,8 +74,8 @@ __device__ __forceinline__ float div_by(float x, float s, float r) {
 }
 
 // RN(1 / s): v_rcp_f32 and one fused correction, equal to the IEEE quotient for every significand
-// (all 2^23 compared on the GPU at eight exponents from -30 to 30; v_rcp_f32 alone differs for
-// 897,675 of them)
+// (tests/test_gpu_append_division.py compares all 2^23 at eight exponents from -30 to 29; v_rcp_f32
+// alone differs for 897,675 of them)
 __device__ __forceinline__ float recip(float s) {
   const float r = __builtin_amdgcn_rcpf(s);
   return fmaf(fmaf(-s, r, 1.0f), r, r);
@@ -524,6 +525,13 @@ __global__ __launch_bounds__(kBulkMaxWaves * 64) void append_bulk_kernel(AppendD
   }
 }
 
+__global__ void division_kernel(const float* x, const float* s, float* r, float* q, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  r[i] = recip(s[i]);
+  q[i] = div_by(x[i], s[i], r[i]);
+}
+
 // the side's format, TILE32 apart from rows
 constexpr int kTileAsym = 7;
 int side_code(const AppendDev& d) { return d.tile32 ? kTileAsym : d.fmt; }
@@ -627,3 +635,14 @@ void append_bulk(const AppendDev& k, const AppendDev& v, const BulkPlan& p, hipS
 }
 
 }  // namespace kvq
+
+extern "C" int kvq_append_division(const float* x, const float* s, float* r, float* q, int64_t n,
+                                   kvq_stream_t stream) {
+  using namespace kvq;
+  if (!x || !s || !r || !q || n < 0 || n > ((int64_t)1 << 31)) return fail(KVQ_ERR_INVALID, "division: bad argument");
+  if (n == 0) return KVQ_OK;
+  hipLaunchKernelGGL(division_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), x, s, r, q, n);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? KVQ_OK : fail(KVQ_ERR_LAUNCH, std::string("launch: ") + hipGetErrorString(e));
+}

@@ -37,6 +37,10 @@ int kvq_dequant(const kvq_kv_view* k, int32_t k_format, int32_t k_group, void* k
 // plan[2] waves a work-group; plan[3] work-groups a side.
 int kvq_append_plan(const kvq_append_params* k, const kvq_append_params* v, int32_t* plan);
 
+// The tile append's division, for its test: r[i] = 1 / s[i] and q[i] = x[i] / s[i] by way of r[i], n
+// device floats each, s within [2^-30, 2^30].
+int kvq_append_division(const float* x, const float* s, float* r, float* q, int64_t n, kvq_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
