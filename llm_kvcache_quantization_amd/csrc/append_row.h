@@ -235,7 +235,6 @@ __device__ __forceinline__ float int4_scale(const AppendDev& a, float stv, float
   return fmaxf(s, 1e-5f);                                      // int4_basic.py:154
 }
 
-// dyn_abs: the group's absmax, or with a percentile its fp32 quantile of |x|
 // dyn_abs: the group's absmax, or with a percentile its fp32 quantile of |x|; stv: the static
 // scale of the group (ld_static; unused without a static table)
 __device__ __forceinline__ half_t int8_scale16(const AppendDev& a, float stv, float dyn_abs) {

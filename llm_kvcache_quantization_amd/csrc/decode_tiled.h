@@ -1679,7 +1679,7 @@ struct KTokT {
   using QInT = QIn;
   static constexpr bool kAppend = false;
   // the writer runs quant_row_x (fused step); with INT4_SYM sides it also finds the group
-  // rescue's threshold over every row of the append (rescue_thr_wave)
+  // rescue's threshold over every row of the append (rescue_thr_rows)
   static constexpr bool kAppendRow = !SH;
   static constexpr bool kRescue = I4;
   static constexpr bool kRowArgs = true;  // the prologue reads most argument lines
@@ -2107,7 +2107,7 @@ __device__ __forceinline__ void append_store(const DecodeArgs& a, const KF& kf, 
 // side of the one-token append exactly as kvq_quant_append's kernel does (quant_row_x on
 // row b * H + h), codes, per-token scales and status words included.  An INT4 side with the
 // group rescue first finds its threshold over every row of the append on its own
-// (rescue_thr_wave: the host admits only thresholds within the walk's reach of the top).
+// (rescue_thr_rows: the host admits only thresholds within the walk's reach of the top).
 __device__ __forceinline__ bool rescue_side(const AppendDev& d) {
   return d.fmt == KVQ_FMT_INT4_SYM && d.st != nullptr && d.rq > 0.f && !d.rescue_all;
 }

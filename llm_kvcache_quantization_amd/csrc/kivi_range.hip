@@ -1,7 +1,8 @@
 // Per-channel ranges of a prompt's K (the frozen parameters of the KIVI layout).
 //
 // Percentiles, and min / max up to range_splits: one work-group takes 8 channels of one (b, head)
-// over all tokens, so nothing is merged between work-groups and the whole reduction is one launch: a thread reads 16 bytes of a token's row.
+// over all tokens, so nothing is merged between work-groups and the whole reduction is one launch: a
+// thread reads 16 bytes of a token's row.
 // The 16 work-groups of a (b, head) run on one XCD (work-group ids go round the 8 XCDs), whose L2
 // then fetches each row once for all of them.
 //

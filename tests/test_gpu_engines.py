@@ -4,7 +4,7 @@
   clip_percentile=99.9 without static scales): codes and scales bit-exact.
 * The calibration tables the reference ships for Qwen2.5-1.5B (group 16; INT8 tables in
   fp16, INT4 tables in fp32 with outlier rescue ratio 0.01; tests/golden/calib_*.json):
-  appends bit-exact through prefill (the rescue's radix select) and decode (its LDS sort),
+  appends bit-exact through prefill (the rescue's key select) and decode (the fused step's writer),
   then decode attention with the tables' inv_tau within max-abs 2e-3 / cosine 0.9999.
 * get_kv / to_tuple / from_tuple against the oracle's dequantizers.
 * Decode steps through append_decode_attn, whose kernel parameters and workspace are kept
@@ -173,8 +173,8 @@ def test_shipped_int8_tables(layer):
 def test_shipped_int4_tables_with_rescue(layer):
     """kv_mode int4_fused with the reference's own table: static fp32 scales, group 16,
     int4_outlier_ratio 0.01 (per-token fp32 scales; the prefill's rescue threshold over
-    2 x 2 x 300 x 8 = 9600 group scales comes from the radix select, the decode steps' from
-    the in-launch sort)."""
+    2 x 2 x 300 x 8 = 9600 group scales comes from the key select, the decode steps' from
+    the fused launch's writer wave)."""
     K = _k()
     t = _shipped(4)
     assert t.group_size == 16 and t.k_scale.dtype == torch.float32 and t.outlier_ratio == 0.01
