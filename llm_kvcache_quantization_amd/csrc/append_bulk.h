@@ -16,14 +16,15 @@ constexpr int kBulkMinTokens = 8;
 constexpr int kBulkTiles32 = 2048, kBulkTiles16 = 512;
 // Tiles for which a work-group has 8 waves instead of 4 where a side counts clipped values (a static
 // table and a status word).  A work-group that clipped adds to the side's one status word and such
-// atomics queue (about 10 ns each), so half as many help as long as about every tile clips and has a
-// wave of its own; a count that stays 0 only pays for the coarser grid.  us for 4 / 8 waves, INT8
-// tables that clip half of the values, and tables that clip none: 1056 tiles 9.6 / 8.9 and 7.8 / 8.7,
-// 1504 10.9 / 9.9 and 8.2 / 8.9, 1952 13.2 / 11.4 and 9.5 / 9.2, 3000 18.3 / 14.3 and 12.2 / 12.1, 8128
-// 60.6 / 44.9 and 44.2 / 44.7, 12000 73.0 / 64.6 and 58.9 / 59.7, 14016 72.4 / 69.6 and 67.2 / 68.0,
-// 20000 90.9 / 91.8 and 89.7 / 92.3.  Sides that count nothing keep 4: INT8 with the 99.9 percentile
-// 2112 tiles 20.6 / 23.2, 4096 30.9 / 31.9, 8128 51.2 / 53.2; the mixed cache 2112 22.6 / 26.2.
-constexpr int kBulkWideFrom = 1728, kBulkWideTo = 13000;
+// atomics queue (about 10 ns each), so half as many help where about every tile clips; a count that
+// stays 0 only pays for the coarser grid.  us for 4 / 8 waves, INT8 tables that clip half of the values,
+// and tables that clip none: 1056 tiles 9.6 / 8.9 and 7.8 / 8.7, 1504 10.9 / 9.9 and 8.2 / 8.9, 1952
+// 13.2 / 11.4 and 9.5 / 9.2, 3000 18.3 / 14.3 and 12.2 / 12.1, 8128 60.6 / 44.9 and 44.2 / 44.7.  Above
+// kBulkWaveSlots a wave takes several tiles; clipping sides still gain there for a while (12000 73.0 /
+// 64.6), those that clip nothing lose (8 bits of KIVI, 10016 tiles 60.7 / 63.5, 14016 71.5 / 78.8).
+// Sides that count nothing keep 4: INT8 with the 99.9 percentile 2112 tiles 20.6 / 23.2, 4096 30.9 /
+// 31.9, 8128 51.2 / 53.2; the mixed cache 2112 22.6 / 26.2.
+constexpr int kBulkWideFrom = 1728, kBulkWideTo = kBulkWaveSlots;
 
 // Order statistics of a percentile (ranks and weight, as torch.quantile computes them) and
 // whether a static table has a per-token policy.

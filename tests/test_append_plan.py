@@ -89,7 +89,7 @@ def test_grid_covers_the_tiles():
 
 def test_waves_a_work_group():
     """8 where a side counts clipped values and the tiles lie in the measured range, else 4."""
-    for S, wide in ((2048, False), (4096, True), (49152, True), (65536, False)):  # 1024, 2048, 12288, 16384 tiles
+    for S, wide in ((2048, False), (4096, True), (32704, True), (32768, False)):  # 1024, 2048, 8176, 8192 tiles
         for k, v, counts in ((_side(I8, S=S, table=True), _side(I8, S=S, table=True), True),
                              (_side(I8, S=S), _side(I8, S=S, table=True), True),
                              (_side(K4, S=S, table=True), _side(K4, S=S), True),
